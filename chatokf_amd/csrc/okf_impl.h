@@ -9,6 +9,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstdint>
+#include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <new>
@@ -22,6 +23,7 @@
 #include "okf_gemv.h"
 #include "okf_gemv_wide.h"
 #include "okf_gemv_sb.h"
+#include "okf_gemm_mm.h"
 #include "okf_ffn.h"
 #include "okf_ffn_mfma.h"
 
@@ -50,18 +52,20 @@ struct okf_ctx {
     int gemv_sb_rw = 0;  // its rows per workgroup (0 = auto)
     int gemv_sb_t = 0;   // its threads per workgroup (0 = auto)
     int gemv_sb_r = 2;   // its rows per lane for IQ2_XXS (2: each x record read serves two rows; or 1)
-    int gemm_ks = 0;     // wide-tile GEMM: K ranges per remainder tile (0 = auto)
+    int gemm_ks = 0;     // tile GEMM: the many-token kernel with this many K ranges (0 = auto)
     int q4k_mm = 0xFFF;  // 2..4 columns on the matrix cores, bits mm_bit(F) (0: the dot4 kernels)
-    int gemm_split = 1;  // tile GEMM of the other formats: K split when the grid is small (0 never, > 1 ways)
-    int gemm_xh = 1;     // tile GEMM of the other formats: fp16 X converted once from N = 256 (0: never)
-    int gemm_thin = 0;   // leftover-tile kernel variant (A/B switch)
-    int gemm_ng = 4;     // wide-tile GEMM: N tiles that share an XCD's row blocks
+    int gemm_plan[4] = {0, 0, 0, 0};  // tile GEMM: this kind, fm, fn, K ranges (plan_mm; fm 0: the plan's choice)
+    int gemm_split = 1;  // tile GEMM: K split when the grid is small (0 never)
+    int gemm_xh = 1;     // tile GEMM of the formats but Q4_K: fp16 X converted once (0: gemm_mfma_kernel on the same
+                         // K ranges, for comparison)
     uint32_t cus = 256;  // compute units of the device
     double fault_rate = 0;
     uint64_t fault_state = 0;
     int last_hip = 0;
     _Float16 *xh = nullptr;  // fp16 copy of the GEMM activations (grown on demand)
     size_t xh_bytes = 0;
+    bool captured = false;          // a captured graph holds scratch addresses: replaced buffers are
+    std::vector<void *> retired;    // kept here until the context is destroyed
     // okf_parallel_begin .. okf_parallel_end: recorded matvecs
     struct Pending {
         int32_t type;
@@ -554,7 +558,16 @@ inline int grow_buf(okf_ctx *c, void **buf, size_t &bytes, size_t need, bool zer
     if (*buf) {
         e = hipStreamSynchronize(c->stream);
         if (e != hipSuccess) return optional ? ((void)hipGetLastError(), OKF_E_HIP) : hip_fail(c, e);
-        (void)hipFree(*buf);
+        bool keep = false;
+        if (c->captured) {
+            try {
+                c->retired.push_back(*buf);
+                keep = true;
+            } catch (const std::bad_alloc &) {
+                return OKF_E_ARG;  // (the buffer stays as it is)
+            }
+        }
+        if (!keep) (void)hipFree(*buf);
         *buf = nullptr;
         bytes = 0;
     }
@@ -587,107 +600,149 @@ inline int grow_xh(okf_ctx *c, size_t need, bool optional = false) {
     return grow_buf(c, (void **)&c->xh, c->xh_bytes, need, false, optional);
 }
 
-// The wide-tile Q4_K GEMM (gemm_q4k_w8_kernel): one 256 x 128 tile per CU.
-// Whole rounds of `cus` tiles stay whole; each remaining tile is split over
-// 16 thin pieces of 64 rows x 32 tokens (gemm_q4k_thin_kernel), or, with
-// OKF_GEMM_KS set, over ks K ranges of whole superblocks
-// (ks * remaining <= cus), whose partial tiles gemm_split_sum_kernel adds in
-// K order.
-inline int launch_gemm_q4k_w(okf_ctx *c, const uint8_t *W, uint64_t rb, uint32_t K, uint32_t M, uint32_t N,
-                      float *Y) {
-    const uint32_t tm = (M + QW_BM - 1) / QW_BM, tn = (N + QG_BN - 1) / QG_BN, sbs = K / 256;
-    GemmSplit sp{};
-    sp.tiles_n = tn;
-    sp.tiles = tm * tn;
-    sp.ng = (uint32_t)c->gemm_ng;
-    const uint32_t round = c->cus ? c->cus : 256, rem = sp.tiles % round;
-    sp.full = sp.tiles - rem;
-    sp.ks = rem ? std::min(c->gemm_ks > 0 ? (uint32_t)c->gemm_ks : round / rem, sbs) : 1;
-    if (sp.ks < 2) {
-        sp.full = sp.tiles + 7 & ~7u;  // no split: every tile whole
-        sp.ks = 1;
-    } else if (c->gemm_ks == 0) {
-        // the leftover tiles as 16 thin pieces each (gemm_q4k_thin_kernel)
-        if (sp.full) {
-            sp.ks = 1;
-            sp.full_xcd = sp.full / 8;
-            hipLaunchKernelGGL((gemm_q4k_w8_kernel<2, 2>), dim3(sp.full), dim3(512), 0, c->stream, W, rb, K, M,
-                               (const _Float16 *)c->xh, N, Y, sp);
+// ---------------------------------------------------------- tile GEMM plan
+// How a tile GEMM runs: the few-token kernel (gemm_few_kernel, kind 0: fm
+// row tiles and fn token tiles of 16 a workgroup) or the many-token one
+// (gemm_many_kernel, kind 1: 16 fm rows x 128 fn tokens), and the K ranges
+// (kper k each).
+struct MmPlan {
+    int kind, fm, fn;
+    uint32_t ks, kper;
+};
+
+// The many-token instances: fm x fn accumulators of 4 registers a lane.
+#define OKF_MANY(X) X(4, 1) X(5, 1) X(6, 1) X(8, 1) X(9, 1) X(4, 2) X(5, 2) X(6, 2) X(8, 2) X(9, 2) X(4, 3) X(5, 3) X(6, 3)
+#define OKF_FEW(X) X(1, 1) X(2, 1) X(1, 2) X(2, 2) X(1, 4) X(2, 4)
+
+inline bool mm_instance(int kind, int fm, int fn) {
+#define OKF_IS(a, b) (fm == a && fn == b) ||
+    return kind == 1 ? OKF_MANY(OKF_IS) false : kind == 0 ? OKF_FEW(OKF_IS) false : false;
+#undef OKF_IS
+}
+
+// The plan with the least estimated time (us), from figures measured on
+// MI355X over 300 x 768 .. 17408 x 5120 and 6 .. 1024 tokens (Q4_K, IQ4_NL):
+//  many: a chunk takes 0.9 + 0.195 fm fn, a workgroup 3.5 besides, one
+//    workgroup a CU at a time (so the tile height that just fills the CUs
+//    wins: 17408 x 5120, N = 101: fm 5 38 us, 4 58, 8 58; N = 512: fm 9, fn 2
+//    88 us, 8, 2 142);
+//  few: a wavefront's step takes 0.4 + 0.17 fm fn, times the workgroups that
+//    share a CU, and 2.5 besides (6144 x 2048, N = 19: 7.7 us against 11.1
+//    for many; N = 48: 10.3 against 13.4);
+//  K ranges: the partial tiles written and read at 4 TB/s, and a launch.
+// From 256 tokens on the formats but Q4_K take only many, whose sums are in
+// gemm_mfma_kernel's order (few takes K in another order within 128).
+inline MmPlan plan_mm(const okf_ctx *c, int type, uint32_t K, uint32_t M, uint32_t N) {
+    const uint32_t cus = c->cus ? c->cus : 256;
+    auto up = [](uint64_t a, uint64_t b) { return (a + b - 1) / b; };
+    MmPlan p{};
+    double best = 0;
+    const int *force = c->gemm_plan;  // (measurements and tests)
+    auto consider = [&](int kind, int fm, int fn, uint32_t ks) {
+        if (force[1] && (kind != force[0] || fm != force[1] || fn != force[2])) return;
+        if (force[1]) ks = (uint32_t)force[3];
+        const uint32_t unit = kind ? MC_BK : 128, steps = (uint32_t)up(K, unit);
+        const uint32_t per = (uint32_t)up(steps, std::max(1u, std::min(ks, steps)));
+        ks = (uint32_t)up(steps, per);
+        const uint64_t wgs = up(M, 16 * fm) * up(N, (kind ? 128 : 16) * fn) * ks;
+        double t = ks > 1 ? 2.5 + (double)ks * N * M * 8 / 4e6 : 0;
+        if (kind) t += (double)up(wgs, cus) * (per * (0.9 + 0.195 * fm * fn) + 3.5);
+        else t += 2.5 + std::max(1.0, (double)wgs / cus) * (double)up(per, 4) * (0.4 + 0.17 * fm * fn);
+        if (best == 0 || t < best) {
+            best = t;
+            p = MmPlan{kind, fm, fn, ks, per * unit};
         }
-        auto thin = [&](auto kern, uint32_t nw) {
-            hipLaunchKernelGGL(kern, dim3((rem * 16 + 7) & ~7u), dim3(nw * 64), 0, c->stream, W, rb, K, M,
-                               (const _Float16 *)c->xh, N, Y, sp.full, tn, rem * 16);
-        };
-        switch (c->gemm_thin) {
-            case 1: thin(gemm_q4k_thin_kernel<8, 2>, 8); break;
-            case 2: thin(gemm_q4k_thin_kernel<8, 4>, 8); break;
-            case 3: thin(gemm_q4k_thin_kernel<4, 2>, 4); break;
-            case 5: thin(gemm_q4k_thin_kernel<4, 6>, 4); break;
-            default: thin(gemm_q4k_thin_kernel<4, 4>, 4); break;
-        }
-        return OKF_OK;
+    };
+    if (force[1] || (c->gemm_ks == 0 && (N < 256 || type == Q4_K))) {
+#define OKF_CONSIDER(a, b)                      \
+    for (uint32_t ks = 1; ks <= 4; ks *= 2) consider(0, a, b, ks);
+        OKF_FEW(OKF_CONSIDER)
+#undef OKF_CONSIDER
     }
-    sp.full_xcd = sp.full / 8;
-    sp.units = sp.ks > 1 ? rem * sp.ks : 0;
-    sp.units_xcd = (sp.units + 7) / 8;
-    if (sp.units) {
-        const int st = grow_part(c, (size_t)sp.units * QW_BM * QG_BN * sizeof(float));
-        if (st) return st;
-        sp.part = c->part;
-    }
-    const uint32_t grid = 8 * (sp.full_xcd + sp.units_xcd);
-    hipLaunchKernelGGL((gemm_q4k_w8_kernel<2, 2>), dim3(grid), dim3(512), 0, c->stream, W, rb, K, M,
-                       (const _Float16 *)c->xh, N, Y, sp);
-    if (sp.units)
-        hipLaunchKernelGGL(gemm_split_sum_kernel<QW_BM>, dim3((sp.tiles - sp.full) * (QW_BM * QG_BN / 1024)),
-                           dim3(256), 0, c->stream, (const float *)c->part, Y, M, N, sp);
-    return OKF_OK;
+    auto many = [&](int fm, int fn) {
+        const uint64_t tiles = up(M, 16 * fm) * up(N, 128 * fn);
+        if (c->gemm_ks > 0) return consider(1, fm, fn, (uint32_t)c->gemm_ks);
+        consider(1, fm, fn, 1);
+        if (!c->gemm_split) return;
+        // as many K ranges as fill one or two rounds of the CUs
+        for (uint32_t r = 1; r <= 2; r++)
+            if (r * cus / tiles > 1) consider(1, fm, fn, (uint32_t)(r * cus / tiles));
+    };
+#define OKF_CONSIDER(a, b) many(a, b);
+    OKF_MANY(OKF_CONSIDER)
+#undef OKF_CONSIDER
+    return p;  // (OKF_GEMM_PLAN is checked against the instances when it is read)
+}
+
+// Marks that a graph being captured now holds the context's scratch
+// addresses: a later growth keeps the old buffer until the context is
+// destroyed.
+inline void note_capture(okf_ctx *c) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c->stream, &cs) != hipSuccess) (void)hipGetLastError();
+    else if (cs != hipStreamCaptureStatusNone) c->captured = true;
 }
 
 template <int F>
 int launch_gemm(okf_ctx *c, const uint8_t *W, uint64_t rb, uint32_t K, uint32_t M, const float *X,
                 uint32_t N, float *Y) {
-    if constexpr (F == Q4_K) {
-        // fp16 activations, converted once per call into the context's buffer
-        const int st = grow_xh(c, (size_t)N * K * sizeof(_Float16));
-        if (st) return st;
-        const uint64_t n4 = (uint64_t)N * K / 4;
-        hipLaunchKernelGGL(x_to_f16_kernel, dim3((uint32_t)((n4 + 256 * XV - 1) / (256 * XV))), dim3(256), 0,
-                           c->stream, X, c->xh, n4);
-        return launch_gemm_q4k_w(c, W, rb, K, M, N, Y);
+    const MmPlan p = plan_mm(c, F, K, M, N);
+    // fp16 activations, converted once per call into the context's buffer
+    // (as octets: x_to_octets_kernel)
+    const int st = c->gemm_xh || F == Q4_K ? grow_xh(c, (size_t)N * K * sizeof(_Float16), F != Q4_K) : OKF_E_SHAPE;
+    if (st && F == Q4_K) return st;
+    uint32_t ks = p.ks, kper = p.kper;
+    if (st && c->gemm_xh) {
+        // no room for them: gemm_mfma_kernel, which rounds X per tile.  A grid
+        // of fewer than two tiles a CU (small M or N) takes K in ks ranges of
+        // whole 64-steps.
+        const uint32_t tiles = ((N + GB_N - 1) / GB_N) * ((M + GB_M - 1) / GB_M), steps = (K + GB_K - 1) / GB_K;
+        ks = 1;
+        if (c->gemm_split != 0 && tiles < 2 * c->cus) {
+            ks = c->gemm_split > 1 ? (uint32_t)c->gemm_split : (2 * c->cus + tiles - 1) / tiles;
+            ks = std::max(1u, std::min(ks, steps / 4));
+        }
+        kper = (steps + ks - 1) / ks * GB_K;
+        ks = (K + kper - 1) / kper;
     }
-    // a grid of fewer than two tiles a CU (small M or N) takes K in ks
-    // ranges of whole 64-steps, partial tiles added by gemm_ksum_kernel
-    // (measured on MI355X, N = 512: Q2_0 2048 x 6144 178 us, Q8_0 2048 x 2048
-    // 72.6 us as one K range); without room for the partials (a reserved
-    // context), one range
-    const uint32_t tiles = ((N + GB_N - 1) / GB_N) * ((M + GB_M - 1) / GB_M), steps = (K + GB_K - 1) / GB_K;
-    uint32_t ks = 1;
-    if (c->gemm_split != 0 && tiles < 2 * c->cus) {
-        ks = c->gemm_split > 1 ? (uint32_t)c->gemm_split : (2 * c->cus + tiles - 1) / tiles;
-        ks = std::max(1u, std::min(ks, steps / 4));
-    }
-    const uint32_t kper = (steps + ks - 1) / ks * GB_K;
-    ks = (K + kper - 1) / kper;
+    // the K ranges' partial tiles, added in K order by gemm_ksum_kernel;
+    // without room for them, one range
     float *part = nullptr;
     if (ks > 1) {
         if (grow_part(c, (size_t)ks * N * M * sizeof(float), true) == OKF_OK) part = c->part;
-        else ks = 1;
+        else ks = 1, kper = (K + MC_BK - 1) / MC_BK * MC_BK;
     }
-    // from N = 256 X is converted to fp16 once (every row tile would round
-    // the same columns again), when the buffer can hold it (measured, us,
-    // N = 512: Q2_0 6144 x 2048 58.9 -> 46.0, 2048 x 6144 52.0 -> 41.8; at
-    // N = 64..128 the extra launch costs about what it saves)
-    const _Float16 *xh = nullptr;
-    if (c->gemm_xh && N >= 256 && K % 32 == 0 && grow_xh(c, (size_t)N * K * sizeof(_Float16), true) == OKF_OK) {
-        const uint64_t n4 = (uint64_t)N * K / 4;
-        hipLaunchKernelGGL(x_to_f16_kernel, dim3((uint32_t)((n4 + 256 * XV - 1) / (256 * XV))), dim3(256), 0,
-                           c->stream, X, c->xh, n4);
-        xh = c->xh;
+    note_capture(c);
+    const u32x4 *tab = dq_tab_rows<F>() ? c->tab8 : nullptr;
+    if (st) {
+        dim3 grid((N + GB_N - 1) / GB_N, (M + GB_M - 1) / GB_M, ks);
+        hipLaunchKernelGGL((gemm_mfma_kernel<F>), grid, dim3(256), 0, c->stream, W, rb, K, M, X, N, Y, c->grid, c->grids,
+                           kper, part);
+    } else {
+        half8 *xt = (half8 *)c->xh;
+        hipLaunchKernelGGL(x_to_octets_kernel, dim3((N + 15) / 16, (K / 8 + 63) / 64), dim3(256), 0, c->stream, X, N, K / 8,
+                           xt);
+        if (p.kind == 0) {
+            auto go = [&](auto fmc, auto fnc) {
+                constexpr int FM = decltype(fmc)::value, FN = decltype(fnc)::value;
+                dim3 grid((M + 16 * FM - 1) / (16 * FM), (N + 16 * FN - 1) / (16 * FN), ks);
+                hipLaunchKernelGGL((gemm_few_kernel<F, FM, FN, 4>), grid, dim3(256), 0, c->stream, W, rb, K, M, xt, N, Y,
+                                   kper / 128, part, tab, c->grid, c->grids);
+            };
+#define OKF_GO(a, b) \
+    if (p.fm == a && p.fn == b) go(std::integral_constant<int, a>{}, std::integral_constant<int, b>{});
+            OKF_FEW(OKF_GO)
+        } else {
+            auto go = [&](auto fmc, auto fnc) {
+                constexpr int FM = decltype(fmc)::value, FN = decltype(fnc)::value;
+                const MmTiles mt{(M + 16 * FM - 1) / (16 * FM), (N + 128 * FN - 1) / (128 * FN), kper / MC_BK};
+                hipLaunchKernelGGL((gemm_many_kernel<F, FM, FN>), dim3(mt.tiles_m * mt.tiles_n, 1, ks), dim3(512), 0,
+                                   c->stream, W, rb, K, M, xt, N, Y, mt, part, tab, c->grid, c->grids);
+            };
+            OKF_MANY(OKF_GO)
+#undef OKF_GO
+        }
     }
-    dim3 grid((N + GB_N - 1) / GB_N, (M + GB_M - 1) / GB_M, ks);
-    hipLaunchKernelGGL((gemm_mfma_kernel<F>), grid, dim3(256), 0, c->stream, W, rb, K, M, X, N, Y,
-                       c->grid, c->grids, ks > 1 ? kper : (steps * GB_K), part, xh);
     if (part) {
         const uint64_t nm = (uint64_t)N * M;
         hipLaunchKernelGGL(gemm_ksum_kernel, dim3((uint32_t)((nm + 1023) / 1024)), dim3(256), 0, c->stream,

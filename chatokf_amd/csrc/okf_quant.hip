@@ -391,8 +391,11 @@ int okf_ctx_create(int device, okf_ctx **out) {
         if (const char *e = getenv("OKF_GEMV_SB_T")) c->gemv_sb_t = atoi(e);
         if (const char *e = getenv("OKF_GEMV_SB_R")) c->gemv_sb_r = atoi(e);
         if (const char *e = getenv("OKF_GEMM_KS")) c->gemm_ks = atoi(e);
-        if (const char *e = getenv("OKF_GEMM_NG")) c->gemm_ng = atoi(e);
-        if (const char *e = getenv("OKF_GEMM_THIN")) c->gemm_thin = atoi(e);
+        if (const char *e = getenv("OKF_GEMM_PLAN")) {
+            int v[4];
+            if (sscanf(e, "%d,%d,%d,%d", v, v + 1, v + 2, v + 3) == 4 && mm_instance(v[0], v[1], v[2]) && v[3] > 0)
+                memcpy(c->gemm_plan, v, sizeof(v));
+        }
         if (const char *e = getenv("OKF_GEMM_SPLIT")) c->gemm_split = atoi(e);
         if (const char *e = getenv("OKF_GEMM_XH")) c->gemm_xh = atoi(e);
         if (const char *e = getenv("OKF_Q4K_MM")) c->q4k_mm = atoi(e);
@@ -423,6 +426,7 @@ int okf_ctx_destroy(okf_ctx *c) {
         (void)hipFree(c->grids);
         (void)hipFree(c->tab);
         (void)hipFree(c->tab8);
+        for (void *p : c->retired) (void)hipFree(p);
         if (c->xh) (void)hipFree(c->xh);
         if (c->part) (void)hipFree(c->part);
         if (c->cnt) (void)hipFree(c->cnt);

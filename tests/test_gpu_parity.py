@@ -1035,3 +1035,35 @@ def test_gguf_upload_then_gemv(enc, tmp_path):
         finally:
             enc.sync()
             enc._lib.okf_gguf_free_device(enc.h, ctypes.c_void_p(base))
+
+
+# ------------------------------------------------------------------ tile GEMM instances
+# Every instance of the two tile GEMM kernels (OKF_GEMM_PLAN: kind, row
+# tiles, token tiles, K ranges; kind 0 gemm_few_kernel, 1 gemm_many_kernel) at
+# rows and tokens that are no multiple of any tile, K with a partial chunk
+# (1184: 32 weights past 4 chunks and 128), one chunk, and several K ranges,
+# against the oracle.  Tolerance: fp16 rounding of both operands, 2^-11 each
+# of the product's 2-norm, as for the tile GEMM above.
+PLANS = [(0, a, b, k) for a, b, k in ((1, 1, 1), (2, 1, 3), (1, 2, 2), (2, 2, 1), (1, 4, 4), (2, 4, 1))] + \
+    [(1, a, b, k) for a, b, k in ((4, 1, 1), (5, 1, 2), (6, 1, 1), (8, 1, 3), (9, 1, 1), (4, 2, 1), (5, 2, 1), (6, 2, 2),
+                                  (8, 2, 1), (9, 2, 2), (4, 3, 1), (5, 3, 1), (6, 3, 2))]
+
+
+@pytest.mark.parametrize("plan", PLANS, ids=lambda p: "-".join(map(str, p)))
+def test_tile_gemm_instances(plan):
+    import os
+    os.environ["OKF_GEMM_PLAN"] = ",".join(map(str, plan))
+    try:
+        e = ok.Enc(0)
+    finally:
+        del os.environ["OKF_GEMM_PLAN"]
+    try:
+        for t, M, K, N in ((Q8_0, 333, 1184, 150), (IQ4_NL, 200, 96, 20), (Q2_0, 150, 1152, 401), (Q4_0, 70, 2080, 9),
+                           (Q4_K, 333, 1280, 150), (Q5_K, 150, 768, 70), (Q6_K, 333, 512, 130), (IQ4_XS, 150, 256, 70),
+                           (IQ2_XXS, 333, 1280, 130), (IQ3_S, 150, 768, 70), (F32, 150, 608, 70)):
+            say("tile instance", plan, NAMES[t], M, K, N)
+            w, X = weights(t, M, K, 25), acts(N, K, 26)
+            ref = oracle.matmul(t, w, K, M, X).astype(np.float64)
+            assert rel(run_gemm(e, t, M, K, w, X, tile=True), ref) <= TOL
+    finally:
+        e.close()
