@@ -172,25 +172,21 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const uint8_t *__rest
 // registers, four K steps of 32 ahead.  One barrier a chunk.
 //
 // LDS half: the 16 bytes of K step kb (of 8), row tile i, octet g (of 4) and
-// row r (of 16) are at kb MC_KS + i MC_TS + g MC_GS + 16 r.  A read takes 16
-// rows of an octet = 256 contiguous bytes per 16 lanes, which is every bank
-// once wherever it starts.  A write instruction's 16 lanes are 8 pieces of two
-// rows, whose octets lie in different K steps or octet columns: with MC_GS
-// 16 bytes past a multiple of the 256 bytes of all banks, and MC_KS 32 bytes,
-// they fall into 16 different places (without the padding, eight lanes met in
-// one bank group, and the writes took a third of the kernel: 17408 x 5120 Q4_K,
-// N = 128: 71.5 us, 47 without them).
-constexpr uint32_t MC_NW = 8, MC_BK = 256, MC_GS = 256 + 16, MC_TS = 4 * MC_GS;
-template <int FM>
-__host__ __device__ constexpr uint32_t mc_stride() {
-    return FM * MC_TS + (256 + 32 - FM * MC_TS % 256) % 256;
-}
-// Row of the 64 that a pass of the workgroup's lanes takes, from lane / 8:
-// in order, but for Q6_K, whose pieces' octets are 16 and 128 bytes apart,
-// with bits 0 and 2 exchanged, so that a write's two rows are 4 apart.
+// row r (of 16) are at 1024 (FM kb + i) + 256 g + 16 (r ^ mc_swz(kb, g)), so a
+// read is 1 KB of which each lane takes 16 bytes, every bank the same number
+// of times.  A write instruction's 16 lanes are 8 pieces of two rows, whose
+// octets lie in different K steps or octet columns, all at the same place of
+// the 256 bytes of all banks but for the exclusive or, which takes the pieces'
+// two rows to 16 different places.  (Unswizzled, the writes took a third of the
+// kernel, 17408 x 5120 Q4_K, N = 128: 71.5 us, 47 without them; padding between
+// the octet columns instead doubled the reads' time.)
+constexpr uint32_t MC_NW = 8, MC_BK = 256;
 template <int F>
-__device__ __forceinline__ uint32_t mc_row(uint32_t p) {
-    return F == Q6_K ? (p & ~5u) | (p & 1) << 2 | ((p >> 2) & 1) : p;
+__device__ __forceinline__ uint32_t mc_swz(uint32_t kb, uint32_t g) {
+    // (bit 3 from kb alone: the lanes of a read that share banks keep apart)
+    if constexpr (F == Q4_K || F == Q5_K) return 4 * (kb >> 1) + 2 * (g >> 1);
+    else if constexpr (F == Q6_K) return 8 * (kb >> 2) + 2 * g;
+    else return 2 * kb;
 }
 
 struct MmTiles {
@@ -203,7 +199,7 @@ __global__ __launch_bounds__(64 * MC_NW, 2) void gemm_many_kernel(
     const uint8_t *__restrict__ W, uint64_t row_bytes, uint32_t K, uint32_t M, const half8 *__restrict__ Xt,
     uint32_t N, float *__restrict__ Y, MmTiles mt, float *__restrict__ part, const u32x4 *__restrict__ tab_g,
     const uint2 *__restrict__ grid, const uint8_t *__restrict__ gt) {
-    constexpr uint32_t TAB = dq_tab_rows<F>(), KS = mc_stride<FM>(), HALF = 8 * KS;
+    constexpr uint32_t TAB = dq_tab_rows<F>(), KS = 1024 * FM, HALF = 8 * KS;
     constexpr uint32_t PIECES = 16 * FM * 8, T = 64 * MC_NW, NP = (PIECES + T - 1) / T;  // a chunk's pieces, and a lane's
     __shared__ __attribute__((aligned(1024))) uint8_t As[2 * HALF];
     __shared__ uint2 tab[TAB ? TAB : 1];
@@ -222,7 +218,7 @@ __global__ __launch_bounds__(64 * MC_NW, 2) void gemm_many_kernel(
         __syncthreads();
     }
     // piece p of a lane: row (T p + t) / 8 of the tile, piece t % 8 of the chunk
-    const uint32_t pj = t & 7, pr = mc_row<F>(t >> 3);
+    const uint32_t pj = t & 7, pr = t >> 3;
     const uint8_t *wrow[NP];
 #pragma unroll
     for (uint32_t p = 0; p < NP; p++) wrow[p] = W + (uint64_t)min(m0 + 8 * MC_NW * p + pr, M - 1) * row_bytes;
@@ -236,11 +232,11 @@ __global__ __launch_bounds__(64 * MC_NW, 2) void gemm_many_kernel(
         const uint32_t u = min(8 * c + pj, units - 1), row = 8 * MC_NW * p + pr;
         half8 h[4];
         dq_piece<F>(raw[p], u, h, tab, grid, gt);
-        uint8_t *base = As + (c & 1) * HALF + MC_TS * (row >> 4) + 16 * (row & 15);
+        uint8_t *base = As + (c & 1) * HALF + 1024 * (row >> 4);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const uint32_t o = dq_octet<F>(pj, i);  // octet of the chunk
-            *(half8 *)(base + (o >> 2) * KS + MC_GS * (o & 3)) = h[i];
+            *(half8 *)(base + (o >> 2) * KS + 256 * (o & 3) + 16 * ((row & 15) ^ mc_swz<F>(o >> 2, o & 3))) = h[i];
         }
     };
     // activations of K step kb (32 k): octet 4 kb + g of the lane's tokens
@@ -271,23 +267,45 @@ __global__ __launch_bounds__(64 * MC_NW, 2) void gemm_many_kernel(
         load_w(c0 + 1, p);
     }
     barrier();
+    // Rows i of K step ks are read one (FN > 1) or two steps ahead, into the
+    // registers of the step just multiplied, across the chunks as well where
+    // the registers allow (CARRY): a chunk's barrier then stands before its
+    // last steps, when every wavefront has their rows in registers and the
+    // next chunk's in LDS.
+    constexpr int PA = FN > 1 ? 1 : 2;
+    constexpr bool CARRY = FM * FN < 18;
+    half8 a[PA][FM];
+    // (computed anew for each step: eight lane offsets kept through the loop
+    // cost the registers that the larger tiles do not have)
+    auto a_at = [&](uint32_t c, int ks) {
+        uint32_t lo = 256 * g + 16 * r16;
+        asm volatile("" : "+v"(lo));
+        const uint32_t sw = mc_swz<F>(ks, F == Q4_K || F == Q5_K || F == Q6_K ? lo >> 8 : 0);
+        return As + (c & 1) * HALF + ks * KS + (lo ^ (16 * sw));
+    };
+    static_assert(2 * NP <= 8 - PA, "the next chunk is in LDS before the barrier");
+    auto read_first = [&](uint32_t c) {
+#pragma unroll
+        for (int k = 0; k < PA; k++)
+#pragma unroll
+            for (int i = 0; i < FM; i++) a[k][i] = *(const half8 *)(a_at(c, k) + 1024 * i);
+    };
+    if (CARRY) read_first(c0);
     for (uint32_t c = c0; c < c1; c++) {
-        const uint8_t *ab = As + (c & 1) * HALF + MC_GS * g + 16 * r16;
         const uint32_t nks = min(8u, units - 8 * c);
         if (nks == 8) {
-            half8 a[FM];
-#pragma unroll
-            for (int i = 0; i < FM; i++) a[i] = *(const half8 *)(ab + MC_TS * i);
+            if (!CARRY) read_first(c);
 #pragma unroll
             for (int ks = 0; ks < 8; ks++) {
+                if (CARRY && ks == 8 - PA) barrier();
+                const uint8_t *an = a_at(ks < 8 - PA ? c : c + 1, (ks + PA) % 8);
 #pragma unroll
                 for (int i = 0; i < FM; i++) {
 #pragma unroll
                     for (int j = 0; j < FN; j++)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], xb[ks % XD][j], acc[i][j], 0, 0, 0);
-                    // the next K step's rows i, into the registers just read:
-                    // the LDS latency hides behind the other rows' products
-                    if (ks < 7) a[i] = *(const half8 *)(ab + (ks + 1) * KS + MC_TS * i);
+                        acc[i][j] =
+                            __builtin_amdgcn_mfma_f32_16x16x32_f16(a[ks % PA][i], xb[ks % XD][j], acc[i][j], 0, 0, 0);
+                    if (CARRY || ks < 8 - PA) a[ks % PA][i] = *(const half8 *)(an + 1024 * i);
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 load_x(8 * c + ks + XD, xb[ks % XD]);
@@ -295,26 +313,26 @@ __global__ __launch_bounds__(64 * MC_NW, 2) void gemm_many_kernel(
                 // of the one after it
 #pragma unroll
                 for (uint32_t p = 0; p < NP; p++)
-                    if (ks == (int)(1 + p * (6 / NP)) && c + 1 < c1) {
+                    if (ks == (int)(2 * p) && c + 1 < c1) {
                         put_w(c + 1, p);
                         load_w(c + 2, p);
                     }
                 __builtin_amdgcn_sched_barrier(0);
             }
+            if (!CARRY) barrier();
         } else {  // the last chunk of a K that is no multiple of 256
             for (uint32_t ks = 0; ks < nks; ks++) {
                 half8 xv[FN];
                 load_x(8 * c + ks, xv);
 #pragma unroll
                 for (int i = 0; i < FM; i++) {
-                    const half8 a = *(const half8 *)(ab + ks * KS + MC_TS * i);
+                    const half8 av = *(const half8 *)(a_at(c, ks) + 1024 * i);
 #pragma unroll
                     for (int j = 0; j < FN; j++)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, xv[j], acc[i][j], 0, 0, 0);
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, xv[j], acc[i][j], 0, 0, 0);
                 }
             }
         }
-        barrier();
     }
     float *dst = part ? part + (uint64_t)blockIdx.z * N * M : Y;
 #pragma unroll

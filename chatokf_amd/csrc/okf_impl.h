@@ -622,14 +622,15 @@ inline bool mm_instance(int kind, int fm, int fn) {
 
 // The plan with the least estimated time (us), from figures measured on
 // MI355X over 300 x 768 .. 17408 x 5120 and 6 .. 1024 tokens (Q4_K, IQ4_NL):
-//  many: a chunk takes 0.9 + 0.195 fm fn, a workgroup 3.5 besides, one
+//  many: a chunk takes fm (0.15 + 0.17 fn), a workgroup 5 besides, one
 //    workgroup a CU at a time (so the tile height that just fills the CUs
 //    wins: 17408 x 5120, N = 101: fm 5 38 us, 4 58, 8 58; N = 512: fm 9, fn 2
-//    88 us, 8, 2 142);
-//  few: a wavefront's step takes 0.4 + 0.17 fm fn, times the workgroups that
-//    share a CU, and 2.5 besides (6144 x 2048, N = 19: 7.7 us against 11.1
-//    for many; N = 48: 10.3 against 13.4);
-//  K ranges: the partial tiles written and read at 4 TB/s, and a launch.
+//    88 us, 8, 2 142), and its outputs, stored by all at once, 5 TB/s;
+//  few: a wavefront's step takes 0.1 + w fm + 0.2 fn + 0.06 fm fn, times the
+//    workgroups that share a CU, and 2.5 besides (6144 x 2048, N = 19: 7.7 us
+//    against 11.1 for many; N = 48: 10.3 against 13.4); w: 0.25, more for the
+//    formats whose pieces take many loads;
+//  K ranges: the partial tiles written and read at 5 TB/s, and a launch.
 // From 256 tokens on the formats but Q4_K take only many, whose sums are in
 // gemm_mfma_kernel's order (few takes K in another order within 128).
 inline MmPlan plan_mm(const okf_ctx *c, int type, uint32_t K, uint32_t M, uint32_t N) {
@@ -637,6 +638,7 @@ inline MmPlan plan_mm(const okf_ctx *c, int type, uint32_t K, uint32_t M, uint32
     auto up = [](uint64_t a, uint64_t b) { return (a + b - 1) / b; };
     MmPlan p{};
     double best = 0;
+    const double w = type == Q6_K ? 0.75 : type == Q8_0 ? 0.6 : dq_fast(type) ? 0.25 : 0.9;
     const int *force = c->gemm_plan;  // (measurements and tests)
     auto consider = [&](int kind, int fm, int fn, uint32_t ks) {
         if (force[1] && (kind != force[0] || fm != force[1] || fn != force[2])) return;
@@ -645,9 +647,9 @@ inline MmPlan plan_mm(const okf_ctx *c, int type, uint32_t K, uint32_t M, uint32
         const uint32_t per = (uint32_t)up(steps, std::max(1u, std::min(ks, steps)));
         ks = (uint32_t)up(steps, per);
         const uint64_t wgs = up(M, 16 * fm) * up(N, (kind ? 128 : 16) * fn) * ks;
-        double t = ks > 1 ? 2.5 + (double)ks * N * M * 8 / 4e6 : 0;
-        if (kind) t += (double)up(wgs, cus) * (per * (0.9 + 0.195 * fm * fn) + 3.5);
-        else t += 2.5 + std::max(1.0, (double)wgs / cus) * (double)up(per, 4) * (0.4 + 0.17 * fm * fn);
+        double t = (double)N * M * 4 / 5e6 + (ks > 1 ? 2.5 + (double)ks * N * M * 8 / 5e6 : 0);
+        if (kind) t += (double)up(wgs, cus) * (per * fm * (0.15 + 0.17 * fn) + 5);
+        else t += 2.5 + std::max(1.0, (double)wgs / cus) * (double)up(per, 4) * (0.1 + w * fm + 0.2 * fn + 0.06 * fm * fn);
         if (best == 0 || t < best) {
             best = t;
             p = MmPlan{kind, fm, fn, ks, per * unit};
