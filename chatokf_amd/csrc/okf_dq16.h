@@ -171,9 +171,7 @@ __device__ __forceinline__ uint32_t iq4_levels_u(uint32_t nib) {
     constexpr uint32_t T0 = iq4_lvu4(0), T1 = iq4_lvu4(4), T2 = iq4_lvu4(8), T3 = iq4_lvu4(12);
     const uint32_t sel = nib & 0x07070707u;
     const uint32_t lo = perm(T1, T0, sel), hi = perm(T3, T2, sel);
-    // 0, 1, 2, 3 for the low half's bytes, 4 .. 7 for the high half's
-    const uint32_t m = ((nib >> 1) & 0x04040404u) | 0x03020100u;
-    return perm(hi, lo, m);
+    return perm(hi, lo, ((nib >> 1) & 0x04040404u) | 0x03020100u);
 }
 
 // Piece r as fp16: h[i] = octet dq_octet(u, i).  tab: the LDS tables

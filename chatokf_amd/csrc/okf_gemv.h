@@ -992,8 +992,8 @@ struct Compute<Q4_0, NC, R, TS> {
 };
 
 // IQ4_NL's 16 levels as int8 bytes (IQ4_NL.kvalues, Gemma4Quant.swift:8-11):
-// a code dword's four low (or high) nibbles index them with two v_perm and a
-// per-byte select on bit 3 (v_perm selector 0x0C gives 0x00, 0x0D 0xFF).
+// a code dword's four low (or high) nibbles index each half of them with one
+// v_perm, and a third takes byte k of the half that bit 3 of nibble k names.
 __host__ __device__ constexpr uint32_t iq4_lvb(int i) { return (uint32_t)(uint8_t)iq4nl_level(i); }
 __host__ __device__ constexpr uint32_t iq4_lv4(int i) {
     return iq4_lvb(i) | iq4_lvb(i + 1) << 8 | iq4_lvb(i + 2) << 16 | iq4_lvb(i + 3) << 24;
@@ -1003,8 +1003,7 @@ struct IQ4Levels {
         constexpr uint32_t T0 = iq4_lv4(0), T1 = iq4_lv4(4), T2 = iq4_lv4(8), T3 = iq4_lv4(12);
         const uint32_t sel = nib & 0x07070707u;
         const uint32_t lo = perm(T1, T0, sel), hi = perm(T3, T2, sel);
-        const uint32_t m = perm(0, 0, ((nib >> 3) & 0x01010101u) | 0x0C0C0C0Cu);
-        return (hi & m) | (lo & ~m);
+        return perm(hi, lo, ((nib >> 1) & 0x04040404u) | 0x03020100u);
     }
 };
 

@@ -1,4 +1,4 @@
-// okf_gemv_sb.h -- matvec with one superblock per lane (Q4_K, IQ2_XXS).
+// okf_gemv_sb.h -- matvec with one superblock (256 weights) per lane.
 //
 // Work items are (row, superblock) pairs.  A workgroup owns RW consecutive
 // rows, i.e. RW * nsb items that lie back to back in memory (GGUF rows are
@@ -34,17 +34,18 @@ constexpr uint32_t SB_CHUNKS = 57;
 
 template <int F>
 __host__ __device__ constexpr bool sb_fmt() {
-    return F == Q4_K || F == IQ2_XXS;
+    return F == Q4_K || F == IQ2_XXS || F == Q5_K || F == IQ4_XS || F == Q4_0 || F == IQ4_NL || F == Q8_0;
 }
-// 16-byte loads a superblock takes, its bytes, and the LDS table rows its
-// compute reads (IQ2_XXS: the grid and sign rows of Compute<IQ2_XXS>)
-template <int F>
-__host__ __device__ constexpr int sb_loads() {
-    return F == Q4_K ? 9 : 5;
-}
+// Bytes of 256 weights, the 16-byte registers they take (IQ2_XXS: d, then
+// four loads from byte 2), and the LDS table rows the compute reads (IQ2_XXS:
+// the grid and sign rows of Compute<IQ2_XXS>)
 template <int F>
 __host__ __device__ constexpr uint32_t sb_bytes() {
-    return F == Q4_K ? 144 : 66;
+    return block_bytes(F) * (256 / block_elems(F));
+}
+template <int F>
+__host__ __device__ constexpr int sb_loads() {
+    return F == IQ2_XXS ? 5 : (sb_bytes<F>() + 15) / 16;
 }
 template <int F>
 __host__ __device__ constexpr uint32_t sb_tab_rows() {
@@ -256,13 +257,114 @@ __device__ __forceinline__ void sb_iq2(const u32x4 (&c)[R][5], const u32x4 *rec,
         for (int n = 0; n < NC; n++) out[r][n] = acc[r][n];
 }
 
+// Dword at byte `off` (a constant) of a superblock's dwords.
+template <int ND>
+__device__ __forceinline__ uint32_t sb_dw(const uint32_t (&c)[ND], uint32_t off) {
+    const uint32_t i = off >> 2;
+    return (off & 3) == 0 ? c[i] : __builtin_amdgcn_alignbyte(c[i + 1], c[i], off & 3);
+}
+// The dwords of a superblock's registers, each a value of its own.  (Taken
+// from the loaded vectors where they are used, hipcc 7.2 -O3 gave the register
+// of IQ4_XS's dword 32 to an address while it was still to be read.)
+template <int NL>
+__device__ __forceinline__ void sb_split(const u32x4 (&c)[NL], uint32_t (&d)[4 * NL]) {
+#pragma unroll
+    for (int k = 0; k < NL; k++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            d[4 * k + i] = c[k][i];
+            asm("" : "+v"(d[4 * k + i]));
+        }
+}
+
+// The other formats, R rows: group j's weights 16 h + 4 k .. + 3 as one dword
+// of int8 (the block layouts of Compute<F> and decode_unit), dotted with the
+// staged planes; the group sum (comb) by f, then the block's scales in the
+// factored form of Compute<F>.  Q4_0 / IQ4_NL / Q8_0: eight 32-weight blocks,
+// 18 or 34 bytes apart.
+template <int F, int R, int NL>
+__device__ __forceinline__ void sb_gen(const u32x4 (&cv)[R][NL], const u32x4 *rec, float (&out)[R][1]) {
+    uint32_t c[R][4 * NL];
+#pragma unroll
+    for (int r = 0; r < R; r++) sb_split(cv[r], c[r]);
+    float acc[R], accm[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) acc[r] = accm[r] = 0.0f;
+    auto bytes = [&](int r, int j, int h, int k) -> uint32_t {
+        if constexpr (F == Q8_0) {
+            return sb_dw(c[r], 34 * j + 2 + 16 * h + 4 * k);
+        } else if constexpr (F == Q4_0 || F == IQ4_NL) {
+            const uint32_t v = (sb_dw(c[r], 18 * j + 2 + 4 * k) >> (4 * h)) & 0x0F0F0F0Fu;
+            return F == Q4_0 ? v : IQ4Levels::levels(v);
+        } else if constexpr (F == IQ4_XS) {
+            return IQ4Levels::levels((sb_dw(c[r], 8 + 16 * j + 4 * k) >> (4 * h)) & 0x0F0F0F0Fu);
+        } else {
+            static_assert(F == Q5_K, "superblock-per-lane format");
+            return ((sb_dw(c[r], 48 + 32 * (j >> 1) + 16 * h + 4 * k) >> (4 * (j & 1))) & 0x0F0F0F0Fu) |
+                   (((sb_dw(c[r], 16 + 16 * h + 4 * k) >> j) & 0x01010101u) << 4);
+        }
+    };
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const floatx4 gd = *(const floatx4 *)&rec[48 + j];
+        int s[3][R][1];
+        zero3(s);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            uint32_t w[R][4];
+#pragma unroll
+            for (int r = 0; r < R; r++)
+#pragma unroll
+                for (int k = 0; k < 4; k++) w[r][k] = bytes(r, j, h, k);
+#pragma unroll
+            for (int p = 0; p < 3; p++) {
+                const u32x4 xv = rec[j * 6 + p * 2 + h];
+#pragma unroll
+                for (int r = 0; r < R; r++)
+#pragma unroll
+                    for (int k = 0; k < 4; k++) s[p][r][0] = sdot4(w[r][k], xv[k], s[p][r][0]);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            if constexpr (F == Q8_0 || F == Q4_0 || F == IQ4_NL) {
+                const uint32_t o = (F == Q8_0 ? 34 : 18) * j;
+                const float d = h2f(c[r][o >> 2] >> (8 * (o & 3)));
+                const float v = comb(s, r, 0) * gd[1];
+                acc[r] = fmaf(d, F == Q4_0 ? v - 8.0f * gd[0] : v, acc[r]);
+            } else if constexpr (F == IQ4_XS) {
+                const uint32_t sh = c[r][0] >> (16 + 2 * j), sl = c[r][1] >> (4 * j);
+                acc[r] = fmaf((float)((int)((sl & 0xF) | (sh & 3) << 4) - 32), comb(s, r, 0) * gd[1], acc[r]);
+            } else if constexpr (F == Q5_K) {
+                const Q4KScales q(u32x4{c[r][0], c[r][1], c[r][2], c[r][3]});
+                acc[r] = fmaf((float)byte_of(q.sc[j >> 2], j & 3), gd[1] * comb(s, r, 0), acc[r]);
+                accm[r] = fmaf((float)byte_of(q.mn[j >> 2], j & 3), gd[0], accm[r]);
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        if constexpr (F == Q5_K) {
+            const Q4KScales q(u32x4{c[r][0], c[r][1], c[r][2], c[r][3]});
+            out[r][0] = q.d * acc[r] - q.dmin * accm[r];
+        } else if constexpr (F == IQ4_XS) {
+            out[r][0] = h2f(c[r][0] & 0xFFFF) * acc[r];
+        } else {
+            out[r][0] = acc[r];
+        }
+    }
+}
+
 // Grid: one workgroup per RW rows of a matrix of the group (GemvGroup as
 // gemv_kernel).  Items are (row pair-set, superblock): item i covers
 // superblock i % nsb of rows i / nsb + k RW / R, k < R (RW a multiple of R).
+// Paired (PAIR; one column, no SiLU staging): the FFN's gate (matrix 0) and
+// up (matrix 1) share x, and a workgroup takes the same RW / 2 rows of both:
+// Y[0] = silu(gate x) (up x), Y[1] = up x, as gemv_body's paired mode.
 // Dynamic LDS: the format's table rows (copied from tab_g), NC columns of
 // nsb records (column stride cs = nsb * SB_CHUNKS chunks), then the
-// partials [row][superblock][NC].
-template <int F, int NC, int R, int T, int SR, bool SILU>
+// partials [row][superblock][NC], and paired the RW row sums.
+template <int F, int NC, int R, int T, int SR, bool SILU, bool PAIR>
 __global__ __launch_bounds__(T) void gemv_sb_kernel(GemvGroup g, uint64_t row_bytes, uint32_t K, uint32_t RW,
                                                     const u32x4 *__restrict__ tab_g) {
     static_assert(sb_fmt<F>(), "no superblock-per-lane matvec for this format");
@@ -270,38 +372,55 @@ __global__ __launch_bounds__(T) void gemv_sb_kernel(GemvGroup g, uint64_t row_by
 #pragma unroll
     for (int k = 0; k + 1 < GV_GROUP; k++)
         if (k + 1 < (int)g.n && blockIdx.x >= g.end[k]) mi = k + 1;
+    static_assert(!PAIR || (NC == 1 && !SILU), "paired: one column, plain staging");
+    if constexpr (PAIR) mi = 0;
     const uint32_t blk = blockIdx.x - (mi ? g.end[mi - 1] : 0);
-    const uint32_t M = g.M[mi];
+    const uint32_t M = g.M[mi], RWH = PAIR ? RW / 2 : RW;
     const float *__restrict__ X = g.X[mi];
     const float *__restrict__ X2 = g.X2[mi];
     float *__restrict__ Y = g.Y[mi];
     extern __shared__ u32x4 lds[];
     const uint32_t tid = threadIdx.x, nsb = K / 256, cs = nsb * SB_CHUNKS;
-    constexpr uint32_t TABR = sb_tab_rows<F>(), NL = sb_loads<F>();
+    constexpr uint32_t TABR = sb_tab_rows<F>();
+    constexpr int NL = sb_loads<F>();
     u32x4 *tab = lds;
     if constexpr (TABR > 0)
         for (uint32_t e = tid; e < TABR; e += T) tab[e] = tab_g[e];
     u32x4 *xs = lds + TABR;
-    float *part = (float *)(xs + NC * cs);
-    const uint32_t r0 = blk * RW, rows = min(RW, M - r0), rs = RW / R;
+    float *part = (float *)(xs + NC * cs), *red = part + RW * nsb * NC;
+    // (paired: rows 0 .. RWH - 1 of the workgroup are gate's, the others up's)
+    const uint32_t r0 = blk * RWH, mrows = min(RWH, M - r0), rows = PAIR ? RW : mrows, rs = RW / R;
     const uint32_t items = rs * nsb;
     const uint8_t *base = g.W[mi] + (uint64_t)r0 * row_bytes;
+    const uint8_t *base2 = PAIR ? g.W[1] + (uint64_t)r0 * row_bytes : base;
 
     u32x4 c[R][NL];
-    auto load = [&](uint32_t it) {
+    auto load = [&](uint32_t it) __attribute__((always_inline)) {
         const uint32_t i = min(it, items - 1), row = i / nsb, sb = i - row * nsb;
 #pragma unroll
         for (int r = 0; r < R; r++) {
             // rows past the matrix re-read the last row (their results are dropped)
-            const uint32_t rr = min(row + r * rs, rows - 1);
-            const uint8_t *p = base + (uint64_t)rr * row_bytes + (uint64_t)sb * sb_bytes<F>();
+            const uint32_t q = row + r * rs;
+            const bool second = PAIR && q >= RWH;
+            const uint32_t rr = min(second ? q - RWH : q, mrows - 1);
+            const uint8_t *p = (second ? base2 : base) + (uint64_t)rr * row_bytes + (uint64_t)sb * sb_bytes<F>();
             if constexpr (F == IQ2_XXS) {
                 c[r][0] = u32x4{ldu<uint16_t>(p), 0u, 0u, 0u};
 #pragma unroll
                 for (int k = 0; k < 4; k++) c[r][1 + k] = ldu<u32x4>(p + 2 + 16 * k);
-            } else {
+            } else if constexpr (F == Q4_K) {
 #pragma unroll
                 for (int k = 0; k < 9; k++) c[r][k] = ((const u32x4 *)p)[k];
+            } else {
+                constexpr int FULL = sb_bytes<F>() / 16;
+#pragma unroll
+                for (int k = 0; k < FULL; k++) c[r][k] = ldu<u32x4>(p + 16 * k);
+                if constexpr (sb_bytes<F>() % 16 == 8) {
+                    const uint2 t = ldu<uint2>(p + 16 * FULL);
+                    c[r][FULL] = u32x4{t.x, t.y, 0u, 0u};
+                } else {
+                    static_assert(sb_bytes<F>() % 16 == 0, "superblock tail");
+                }
             }
         }
     };
@@ -314,7 +433,8 @@ __global__ __launch_bounds__(T) void gemv_sb_kernel(GemvGroup g, uint64_t row_by
         float o[R][NC];
         const uint32_t row = it / nsb, sb = it - row * nsb;
         if constexpr (F == IQ2_XXS) sb_iq2<NC, R>(c, xs + sb * SB_CHUNKS, cs, tab, o);
-        else sb_q4k<NC, R>(c, xs + sb * SB_CHUNKS, cs, o);
+        else if constexpr (F == Q4_K) sb_q4k<NC, R>(c, xs + sb * SB_CHUNKS, cs, o);
+        else sb_gen<F, R, NL>(c, xs + sb * SB_CHUNKS, o);
         if (it + T < items) load(it + T);
 #pragma unroll
         for (int r = 0; r < R; r++)
@@ -336,7 +456,10 @@ __global__ __launch_bounds__(T) void gemv_sb_kernel(GemvGroup g, uint64_t row_by
             for (uint32_t sb = l16; sb < nsb; sb += 16) v += part[(r * nsb + sb) * NC + n];
 #pragma unroll
             for (int m = 1; m < 16; m <<= 1) v += __shfl_xor(v, m, 16);
-            if (l16 == 0) Y[(uint64_t)n * M + r0 + r] = v;
+            if (l16 == 0) {
+                if constexpr (PAIR) red[r] = v;
+                else Y[(uint64_t)n * M + r0 + r] = v;
+            }
         }
     } else {
         const uint32_t lane4 = tid & 3;
@@ -345,7 +468,18 @@ __global__ __launch_bounds__(T) void gemv_sb_kernel(GemvGroup g, uint64_t row_by
             float v = 0.0f;
             for (uint32_t sb = lane4; sb < nsb; sb += 4) v += part[(r * nsb + sb) * NC + n];
             v = quad_sum(v);
-            if (lane4 == 0) Y[(uint64_t)n * M + r0 + r] = v;
+            if (lane4 == 0) {
+                if constexpr (PAIR) red[r] = v;
+                else Y[(uint64_t)n * M + r0 + r] = v;
+            }
+        }
+    }
+    if constexpr (PAIR) {
+        __syncthreads();
+        if (tid < mrows) {
+            const float u = red[RWH + tid];
+            g.Y[0][r0 + tid] = silu_mul1(red[tid], u);
+            g.Y[1][r0 + tid] = u;
         }
     }
 }

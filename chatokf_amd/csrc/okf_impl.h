@@ -349,15 +349,15 @@ bool launch_gemv_wide(okf_ctx *c, const GemvCall &call, uint64_t rb, uint32_t K)
     return true;
 }
 
-template <int F, int NC, int T, bool SILU, int R = 1>
+template <int F, int NC, int T, bool SILU, int R = 1, bool PAIR = false>
 void launch_sb_t(okf_ctx *c, const GemvGroup &g, uint32_t total, uint64_t rb, uint32_t K, uint32_t RW, size_t lds,
                  uint32_t sr) {
     auto go = [&](auto src) {
         constexpr int SR = decltype(src)::value;
-        const void *fn = (const void *)gemv_sb_kernel<F, NC, R, T, SR, SILU>;
+        const void *fn = (const void *)gemv_sb_kernel<F, NC, R, T, SR, SILU, PAIR>;
         static std::atomic<uint64_t> attr{0};  // devices that have the attribute set
         set_lds_attr(c, fn, attr);
-        hipLaunchKernelGGL((gemv_sb_kernel<F, NC, R, T, SR, SILU>), dim3(total), dim3(T), lds, c->stream, g, rb, K,
+        hipLaunchKernelGGL((gemv_sb_kernel<F, NC, R, T, SR, SILU, PAIR>), dim3(total), dim3(T), lds, c->stream, g, rb, K,
                            RW, (const u32x4 *)c->tab8);
     };
     // (one register buffer: a two-deep ring measured slower at every
@@ -372,34 +372,64 @@ void launch_sb_t(okf_ctx *c, const GemvGroup &g, uint32_t total, uint64_t rb, ui
     }
 }
 
+// Where the superblock-per-lane matvec is the faster one, by the superblocks
+// (256 weights) of the call.  Measured on MI355X against gemv_kernel (us,
+// gemv_kernel -> superblock): Q4_K 2048 x 2048 (16 K superblocks) 3.4 -> 4.0,
+// 6144 x 2048 (49 K) 4.4 -> 4.1; Q5_K 2048 x 2048 3.6 -> 4.2, 3000 x 2816 5.5 ->
+// 4.7, 17408 x 5120 16.1 -> 13.3, 5120 x 17408 22.8 -> 15.5; Q8_0 6144 x 2048
+// 4.8 -> 5.1, 5120 x 5120 8.8 -> 7.8, 17408 x 5120 22.8 -> 18.2; IQ4_XS 6144 x
+// 2048 4.8 -> 5.1, 5120 x 5120 8.1 -> 7.7, 5120 x 17408 22.3 -> 16.7; Q4_0 12288 x
+// 3584 (172 K) 7.2 -> 7.7, 17408 x 5120 12.4 -> 11.5, 5120 x 17408 19.9 -> 13.5;
+// IQ4_NL 17408 x 5120 (348 K) 14.9 -> 15.3, 60000 x 2048 18.7 -> 17.0, 5120 x 17408
+// 22.0 -> 17.2; IQ2_XXS 2048 x 2048 4.1 -> 7.6, 12288 x 3584 9.8 -> 11.4, 17408 x 5120
+// 14.9 -> 13.9, 60000 x 2048 15.6 -> 16.6.  Gate and up paired (okf_ffn, H x D):
+// 6144 x 2048 Q4_K 10.6 -> 10.8, Q5_K 11.6 -> 11.9, Q8_0 12.5 -> 13.1; 7168 x 3584 Q4_K
+// 16.4 -> 16.0, Q5_K 20.7 -> 17.7, IQ4_NL 18.3 -> 19.7; 17408 x 5120 Q4_K 37.2 -> 35.8,
+// Q5_K 55.6 -> 41.9, IQ4_XS 50.6 -> 44.9, IQ4_NL 55.6 -> 45.3, Q4_0 52.6 -> 35.7, Q8_0
+// 78.7 -> 59.7, IQ2_XXS 41.3 -> 41.9.
+template <int F>
+bool sb_auto(uint64_t rows, uint32_t K, bool pair) {
+    const uint64_t n = rows * (K / 256);  // (paired: of both matrices)
+    const bool lng = K > 8192;
+    if (pair) return n >= (F == Q4_K || F == Q5_K || F == IQ4_XS ? 190000u : 380000u);
+    switch (F) {
+        case Q4_K: return lng || n >= 30000;
+        case Q5_K: return n >= 30000;
+        case IQ2_XXS: return n >= 100000 && K >= 5120;
+        case Q4_0: return n >= (lng ? 96000u : 300000u);
+        case IQ4_NL: return n >= (lng ? 96000u : 400000u);
+        default: return n >= 96000;  // Q8_0, IQ4_XS
+    }
+}
+
 // Superblock-per-lane matvec (gemv_sb_kernel): true when launched.  Short
 // rows (<= 32 superblocks): T = 256 lanes and RW = T / nsb rows, one
-// superblock per lane (IQ2_XXS: two rows per lane, RW = 2 T / nsb; 17408 x
-// 5120 in 15.5 us against 16.1 for one row per lane and for gemv_kernel).  Long rows: T = 512 and RW = M / CUs (one workgroup
-// per CU, each lane a few superblocks), so that the per-workgroup staging of
-// x is shared by more rows.  Measured on MI355X (A/B in one process):
-// Q4_K 17408 x 5120 from 15.7 us (gemv_kernel) to 13.6 us; 5120 x 17408
-// from 17.6 us (gemv_wide_kernel) to 16.4 us.
+// superblock per lane (IQ2_XXS: two rows per lane, RW = 2 T / nsb).  Long
+// rows: T = 512 and RW = M / CUs (one workgroup per CU, each lane a few
+// superblocks), so that the per-workgroup staging of x is shared by more
+// rows.
 template <int F, int NC, bool SILU>
-bool launch_gemv_sb(okf_ctx *c, const GemvCall *calls, int n, uint64_t rb, uint32_t K) {
-    if constexpr (!sb_fmt<F>() || NC > 1) {
+bool launch_gemv_sb(okf_ctx *c, const GemvCall *calls, int n, uint64_t rb, uint32_t K, bool pair = false) {
+    if constexpr (!sb_fmt<F>() || NC > 1 || (SILU && F != Q4_K && F != IQ2_XXS)) {
         return false;
     } else {
         const uint32_t nsb = K / 256;
-        if (c->gemv_sb == 0) return false;
+        if (c->gemv_sb == 0 || K % 256) return false;
+        uint32_t M = 0;
+        for (int i = 0; i < n; i++) M += calls[i].M;
+        if (c->gemv_sb < 0 && !sb_auto<F>(M, K, pair)) return false;
         const bool lng = nsb > 32;
-        if (F == IQ2_XXS && lng) return false;  // (long rows: gemv_kernel, not measured here)
+        if (F == IQ2_XXS && (lng || pair)) return false;  // (long or paired rows: gemv_kernel is no slower)
         uint32_t T = c->gemv_sb_t ? (uint32_t)c->gemv_sb_t : lng ? 512 : 256;
         if (T != 256 && T != 512) T = 256;
         const uint32_t sr = (K / 8 + T - 1) / T;  // staging rounds
         if (sr > 9) return false;
-        uint32_t M = 0;
-        for (int i = 0; i < n; i++) M += calls[i].M;
-        const uint32_t RW = c->gemv_sb_rw ? (uint32_t)c->gemv_sb_rw
-                            : lng       ? std::min(32u, std::max(4u, (M + c->cus - 1) / c->cus))
-                                        : std::max(1u, T / nsb) * (F == IQ2_XXS && c->gemv_sb_r == 2 ? 2 : 1);
+        uint32_t RW = c->gemv_sb_rw ? (uint32_t)c->gemv_sb_rw
+                      : lng       ? std::min(32u, std::max(4u, (M + c->cus - 1) / c->cus))
+                                  : std::max(1u, T / nsb) * (F == IQ2_XXS && c->gemv_sb_r == 2 ? 2 : 1);
+        if (pair) RW += RW & 1;
         const size_t lds = (size_t)sb_tab_rows<F>() * 16 + ((size_t)NC * nsb * SB_CHUNKS * 16) +
-                           (size_t)RW * nsb * NC * sizeof(float);
+                           (size_t)RW * nsb * NC * sizeof(float) + (pair ? RW * sizeof(float) : 0);
         if (lds > c->max_lds) return false;
         GemvGroup g{};
         uint32_t total = 0;
@@ -413,8 +443,17 @@ bool launch_gemv_sb(okf_ctx *c, const GemvCall *calls, int n, uint64_t rb, uint3
             g.end[i] = total;
         }
         g.n = (uint32_t)n;
-        if (F == IQ2_XXS && c->gemv_sb_r == 2 && T == 256 && RW % 2 == 0)
-            launch_sb_t<F, NC, 256, SILU, 2>(c, g, total, rb, K, RW, lds, sr);
+        if (pair) total = (calls[0].M + RW / 2 - 1) / (RW / 2);
+        const bool two = F == IQ2_XXS && c->gemv_sb_r == 2 && T == 256 && RW % 2 == 0;
+        if constexpr (!SILU)
+            if (pair) {
+                if constexpr (F != IQ2_XXS) {
+                    if (T == 256) launch_sb_t<F, NC, 256, false, 1, true>(c, g, total, rb, K, RW, lds, sr);
+                    else launch_sb_t<F, NC, 512, false, 1, true>(c, g, total, rb, K, RW, lds, sr);
+                }
+                return true;
+            }
+        if (two) launch_sb_t<F, NC, 256, SILU, F == IQ2_XXS ? 2 : 1>(c, g, total, rb, K, RW, lds, sr);
         else if (T == 256) launch_sb_t<F, NC, 256, SILU>(c, g, total, rb, K, RW, lds, sr);
         else launch_sb_t<F, NC, 512, SILU>(c, g, total, rb, K, RW, lds, sr);
         return true;
@@ -517,6 +556,7 @@ template <int F>
 void launch_gemv_pair(okf_ctx *c, const GemvCall *calls, uint64_t rb, uint32_t K) {
     if constexpr (F == Q2_0)
         if (launch_q2m(c, calls[0], &calls[1], rb, K)) return;
+    if (launch_gemv_sb<F, 1, false>(c, calls, 2, rb, K, true)) return;
     constexpr uint32_t UW = unit_weights<F>();
     const size_t tab = gemv_tab_rows<F>() * 16;
     const uint32_t units = K / UW;

@@ -1067,3 +1067,53 @@ def test_tile_gemm_instances(plan):
             assert rel(run_gemm(e, t, M, K, w, X, tile=True), ref) <= TOL
     finally:
         e.close()
+
+
+# ------------------------------------------------------------------ superblock-per-lane matvec
+# gemv_sb_kernel, forced (OKF_GEMV_SB=1) and off (0), at its edges: one row, one
+# superblock, rows that fill no workgroup, short rows (a superblock a lane)
+# and long ones (> 32 superblocks, several a lane), single, grouped and paired
+# with the SiLU.  Against the oracle at the matvec gate, and against the
+# general kernel to 1e-5 (both sum exact integer group products; only the
+# fp32 order of the groups differs).
+@pytest.fixture(scope="module")
+def enc_sb():
+    import os
+    es = []
+    for v in ("1", "0"):
+        os.environ["OKF_GEMV_SB"] = v
+        try:
+            es.append(ok.Enc(0))
+        finally:
+            del os.environ["OKF_GEMV_SB"]
+    yield es
+    for e in es:
+        e.close()
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q5_K, IQ4_XS, Q4_0, IQ4_NL, Q8_0], ids=lambda t: NAMES[t])
+@pytest.mark.parametrize("M,K", [(1, 256), (7, 768), (1001, 2304), (300, 8192), (13, 8448), (700, 10240)])
+def test_gemv_superblock_edges(enc_sb, t, M, K):
+    say("superblock matvec", NAMES[t], M, K)
+    w, X = weights(t, M, K, 27), acts(1, K, 28)
+    ref = oracle.matvec(t, w, K, M, X[0]).astype(np.float64)
+    got, gen = (run_gemm(e, t, M, K, w, X)[0] for e in enc_sb)
+    assert rel(got, ref) <= TOL_MV
+    assert rel(got, gen.astype(np.float64)) <= 1e-5
+    w2 = weights(t, M, K, 29)
+    qg, qu = ok.QuantTensor(dev(w), K, M, t), ok.QuantTensor(dev(w2), K, M, t)
+    outs = []
+    for e in enc_sb:
+        g, u, a, b = (torch.full((M,), float("nan"), device="cuda") for _ in range(4))
+        e.gemv_gate_up(qg, qu, dev(X), g, u)
+        with e.parallel():
+            e.gemv(qg, dev(X), a)
+            e.gemv(qu, dev(X), b)
+        e.sync()
+        outs.append([host(v) for v in (g, u, a, b)])
+    up = oracle.matvec(t, w2, K, M, X[0])
+    want = (oracle.silu_mul(ref.astype(np.float32), up), up, ref, up)
+    for o, r in zip(outs[0], want):
+        assert rel(o, r.astype(np.float64)) <= TOL_MV
+    for o, r in zip(*outs):
+        assert rel(o, r.astype(np.float64)) <= 1e-5
