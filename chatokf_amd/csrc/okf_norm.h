@@ -8,78 +8,97 @@ namespace okf {
 
 constexpr int NORM_THREADS = 256;
 
-// Sum over a workgroup of NORM_THREADS threads (every thread gets it):
-// the wavefront's 64 lanes with cross-lane adds, then the 4 wavefront sums
-// through LDS in wavefront order.
+// Sum over a workgroup of NT threads (every thread gets it): the
+// wavefront's 64 lanes with cross-lane adds, then the wavefront sums through
+// LDS in wavefront order.
+template <int NT>
 __device__ __forceinline__ float block_sum(float v, float *red) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
     const uint32_t w = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0) red[w] = v;
     __syncthreads();
-    const float s = (red[0] + red[1]) + (red[2] + red[3]);
-    __syncthreads();  // red is reused by the next call
+    float s = 0;
+#pragma unroll
+    for (int k = 0; k < NT / 64; k += 4) s += (red[k] + red[k + 1]) + (red[k + 2] + red[k + 3]);
     return s;
 }
 
 // add_rmsnorm_batch (LLM/metal/Kernels.metal:2839-2862) and, with R null,
 // rmsnorm_batch (:2818-2836): per row, x += r (stored back), then
 // y = x * (1 / sqrt(mean(x^2) + eps)) * w, with w fp32 (llama.cpp's
-// build_norm: the stored weight multiplies directly).  One workgroup per
-// row; a row is read once into registers when it fits (n <= 4 * 256 * 8),
-// else read twice.
-template <bool ADD>
-__global__ __launch_bounds__(NORM_THREADS) void add_rmsnorm_kernel(float *X,
-                                                                   const float *__restrict__ R,
-                                                                   const float *__restrict__ Wn,
-                                                                   float *Y, uint32_t n,
-                                                                   float eps) {
-    __shared__ float red[4];
+// build_norm: the stored weight multiplies directly).  One workgroup of NT
+// threads per row; a row is read once into registers when it fits (n <= 4 V
+// NT), else read twice.  AHEAD: every load of the row, w's included, is issued
+// before the first is used, so that nothing is loaded behind the sum.  NT =
+// 1024 where there are fewer rows than CUs (a decode step's one row: a thread
+// waits for one or two loads instead of five): 1 x 5120 3.6 -> 2.6 us, with r
+// 3.8 -> 3.0, 64 x 5120 3.9 -> 2.9.  More rows without r: NT = 512, 512 x 5120 6.2
+// -> 5.2; with r they stream 84 KB a row from memory, and fewer registers a
+// wavefront is what counts: NT = 256, not ahead (1024 x 5120 12.9 us; NT = 512
+// ahead 14.4).
+template <bool ADD, int NT, bool AHEAD>
+__global__ __launch_bounds__(NT) void add_rmsnorm_kernel(float *X, const float *__restrict__ R,
+                                                         const float *__restrict__ Wn, float *Y, uint32_t n,
+                                                         float eps) {
+    __shared__ float red[NT / 64];
     const uint64_t row = blockIdx.x;
     float *x = X + row * n;
     const float *r = R + (ADD ? row * n : 0);
     float *y = Y + row * n;
     const uint32_t tid = threadIdx.x;
-    constexpr uint32_t V = 8;  // float4 per thread kept in registers
+    constexpr uint32_t V = 2048 / NT;  // float4 per thread kept in registers
     const uint32_t n4 = n / 4;
-    floatx4 v[V];
+    floatx4 v[V], w[AHEAD ? V : 1];
     float ss = 0;
-    const bool vec = (n % 4) == 0 && n4 <= V * NORM_THREADS &&
+    const bool vec = (n % 4) == 0 && n4 <= V * NT &&
                      (((uintptr_t)X | (uintptr_t)R | (uintptr_t)Wn | (uintptr_t)Y) & 15) == 0;
     if (vec) {
+        floatx4 a[ADD && AHEAD ? V : 1];
+        if constexpr (AHEAD) {
+#pragma unroll
+            for (uint32_t k = 0; k < V; k++) {
+                const uint32_t i = tid + k * NT;
+                if (i < n4) {
+                    v[k] = ((const floatx4 *)x)[i];
+                    if constexpr (ADD) a[k] = ((const floatx4 *)r)[i];
+                    w[k] = ((const floatx4 *)Wn)[i];
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
         for (uint32_t k = 0; k < V; k++) {
-            const uint32_t i = tid + k * NORM_THREADS;
+            const uint32_t i = tid + k * NT;
             if (i < n4) {
-                floatx4 a = ((const floatx4 *)x)[i];
+                if constexpr (!AHEAD) v[k] = ((const floatx4 *)x)[i];
                 if constexpr (ADD) {
-                    a += ((const floatx4 *)r)[i];
-                    ((floatx4 *)x)[i] = a;
+                    v[k] += AHEAD ? a[k % (AHEAD ? V : 1)] : ((const floatx4 *)r)[i];
+                    ((floatx4 *)x)[i] = v[k];
                 }
-                v[k] = a;
-                ss += a[0] * a[0] + a[1] * a[1] + a[2] * a[2] + a[3] * a[3];
+                ss += v[k][0] * v[k][0] + v[k][1] * v[k][1] + v[k][2] * v[k][2] + v[k][3] * v[k][3];
             }
         }
     } else {
-        for (uint32_t i = tid; i < n; i += NORM_THREADS) {
-            float a = x[i];
+        for (uint32_t i = tid; i < n; i += NT) {
+            float b = x[i];
             if constexpr (ADD) {
-                a += r[i];
-                x[i] = a;
+                b += r[i];
+                x[i] = b;
             }
-            ss += a * a;
+            ss += b * b;
         }
     }
-    const float scale = 1.0f / sqrtf(block_sum(ss, red) / (float)n + eps);
+    const float scale = 1.0f / sqrtf(block_sum<NT>(ss, red) / (float)n + eps);
     if (vec) {
 #pragma unroll
         for (uint32_t k = 0; k < V; k++) {
-            const uint32_t i = tid + k * NORM_THREADS;
-            if (i < n4) ((floatx4 *)y)[i] = v[k] * scale * ((const floatx4 *)Wn)[i];
+            const uint32_t i = tid + k * NT;
+            if (i < n4) ((floatx4 *)y)[i] = v[k] * scale * (AHEAD ? w[k % (AHEAD ? V : 1)] : ((const floatx4 *)Wn)[i]);
         }
     } else {
         // (each thread re-reads only the elements it wrote itself)
-        for (uint32_t i = tid; i < n; i += NORM_THREADS) y[i] = x[i] * scale * Wn[i];
+        for (uint32_t i = tid; i < n; i += NT) y[i] = x[i] * scale * Wn[i];
     }
 }
 

@@ -558,12 +558,12 @@ int okf_add_rmsnorm_batch(okf_ctx *c, float *x, const float *r, const float *w, 
     if (n == 0 || rows == 0) return OKF_E_SHAPE;
     int st = begin(c);
     if (st) return st;
-    if (r)
-        hipLaunchKernelGGL(add_rmsnorm_kernel<true>, dim3(rows), dim3(NORM_THREADS), 0, c->stream, x, r, w, y,
-                           n, eps);
-    else
-        hipLaunchKernelGGL(add_rmsnorm_kernel<false>, dim3(rows), dim3(NORM_THREADS), 0, c->stream, x, r, w,
-                           y, n, eps);
+    auto go = [&](auto kern, uint32_t nt) {
+        hipLaunchKernelGGL(kern, dim3(rows), dim3(nt), 0, c->stream, x, r, w, y, n, eps);
+    };
+    const bool few = rows < c->cus;  // (fewer rows than CUs: more threads a row)
+    if (r) few ? go(add_rmsnorm_kernel<true, 1024, true>, 1024) : go(add_rmsnorm_kernel<true, 256, false>, 256);
+    else few ? go(add_rmsnorm_kernel<false, 1024, true>, 1024) : go(add_rmsnorm_kernel<false, 512, true>, 512);
     return finish(c);
 }
 
