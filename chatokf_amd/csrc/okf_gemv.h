@@ -1430,9 +1430,26 @@ struct GemvGroup {
     uint32_t pair;  // 1: W[0] (gate) and W[1] (up) paired in each workgroup (gemv_body)
 };
 
+// Wavefronts a workgroup of gemv_kernel may have: four for one column.  With
+// more columns the staged x leaves room for one workgroup of long rows per CU,
+// and four wavefronts are too few to hide the LDS reads of one another: twelve
+// where the kernel's registers allow (168 each), else eight (256).  Q4_K and
+// Q5_K with four and five columns take all 512 and stay at four.
+template <int F, int NC>
+__host__ __device__ constexpr uint32_t gemv_max_waves() {
+    if (NC == 1) return 4;
+    if (F == Q4_K || F == Q5_K) return NC >= 4 ? 4 : NC == 2 && F == Q4_K ? 12 : 8;
+    if (F == Q3_K) return 8;
+    if (NC == 5) return F == Q8_0 ? 12 : 8;
+    if (NC == 4) return F == F32 || F == F16 || F == Q2_K || F == IQ3_S || F == BF16 ? 8 : 12;
+    return 12;
+}
+
 template <int F, int NC, int R, int D, int S, bool SILU>
-__global__ __launch_bounds__(256) void gemv_kernel(GemvGroup g, uint64_t row_bytes, uint32_t K,
-                                                   const u32x4 *__restrict__ tab_g, uint32_t cunits) {
+__global__ __launch_bounds__((64 * gemv_max_waves<F, NC>())) void gemv_kernel(GemvGroup g, uint64_t row_bytes,
+                                                                              uint32_t K,
+                                                                              const u32x4 *__restrict__ tab_g,
+                                                                              uint32_t cunits) {
     uint32_t i = 0;
 #pragma unroll
     for (int k = 0; k + 1 < GV_GROUP; k++)

@@ -174,30 +174,84 @@ inline int finish(okf_ctx *c) {
     return e == hipSuccess ? OKF_OK : hip_fail(c, e);
 }
 
+// Rows per slot of gemv_kernel: two (each staged activation read serves both)
+// where measured faster: IQ2_XXS with 1..5 columns (16.9 -> 16.4 us at one),
+// the generic formats with 2..5 (17408 x 5120, N = 4: 15-18 % faster; at one
+// column 10-25 % slower), Q4_K and Q2_0 with 5.  (A three-deep ring for the
+// Q4_K matvec measured 3-4 % slower than two once the weight loads were issued
+// behind the staging's.)
+template <int F, int NC>
+constexpr int gemv_rows() {
+    return ((F == IQ2_XXS && NC >= 1) || (grid_fmt(F) && NC >= 2) ||
+            (NC == 5 && F != Q8_0 && F != Q5_K && F != Q6_K && F != IQ4_XS)) ? 2 : 1;
+}
+
+// The workgroup of gemv_kernel for 2..5 columns: its wavefronts W and the K
+// split S over them (W / S * GV_SLOTS * R rows), by an estimated time in us
+// fitted to MI355X at 2048 x 6144 to 17408 x 5120.  A round of workgroups costs
+// its staging and latency plus its rows; workgroups that share a CU (LDS, and
+// its wavefronts' registers) add their rows; wavefronts that do not divide over
+// the four SIMDs, or fewer than eight on a CU, slow the rows down.  Against
+// four wavefronts and no split everywhere (us, N = 2 / 3 / 4 / 5):
+//   5120 x 17408   Q4_0 34.6 / 48.1 / 60.8 / 47.7 -> 18.0 / 24.6 / 30.5 / 43.9,
+//                  Q8_0 40.0 / 51.2 / 62.0 / 73.5 -> 25.2 / 28.7 / 32.9 / 40.0
+//   4096 x 14336   IQ3_XXS 24.5 / 31.3 / 40.0 / 43.7 -> 16.4 / 21.3 / 25.4 / 28.9
+//   17408 x 5120   Q6_K 26.1 / 45.4 / 54.8 / 62.2 -> 22.0 / 30.1 / 36.2 / 51.9
+//   2048 x 6144    IQ4_XS 9.2 / 11.1 / 13.2 / 15.3 -> 7.2 / 8.7 / 10.0 / 11.4
+//   2048 x 2048    Q8_0 4.5 / 5.3 / 6.1 / 7.0 -> 4.2 / 4.9 / 5.5 / 6.1
+struct GemvPlan {
+    uint32_t W, S;
+    float us;
+};
+template <int F, int NC>
+GemvPlan plan_gemv(const okf_ctx *c, uint64_t M, uint32_t K) {
+    constexpr uint32_t R = gemv_rows<F, NC>(), MAXW = gemv_max_waves<F, NC>(), L = GV_L;
+    constexpr uint8_t forms[][2] = {{4, 1}, {8, 1}, {10, 1}, {12, 1}, {4, 2}, {6, 2},
+                                    {8, 2}, {10, 2}, {12, 2}, {4, 4}, {8, 4}, {12, 4}};
+    const uint32_t steps = (K / unit_weights<F>() + L - 1) / L;
+    const size_t xb = (size_t)NC * K / unit_weights<F>() * unit_lds_bytes<F>() + gemv_tab_rows<F>() * 16;
+    const float k = K / 14336.0f, stage = 0.5f + k * (2.3f + 2.05f * NC), row = k * (0.17f + 0.13f * NC);
+    GemvPlan best{4, 1, 1e30f};
+    // (many short rows: small workgroups, several on a CU, stage while others
+    // compute; Q8_0 N = 2 at 30000 x 2048 14.4 us, with larger ones 17.9; at
+    // 20000 x 4096 17.5 against 18.9)
+    const bool many = !c->gemv_s && K <= 4096 && M > 64ull * c->cus;
+    for (const auto &f : forms) {
+        const uint32_t W = f[0], S = f[1], rows = W / S * GV_SLOTS * R;
+        if (many && (W > 4 || S > 1)) continue;
+        if (F == Q6_K && steps < 2 * S) continue;  // (2048 x 2048, N = 3: 5.5 us without a split, 5.9 with)
+        if (W > MAXW || (c->gemv_s && S != std::min<uint32_t>(c->gemv_s, 4))) continue;
+        const uint32_t fit = (uint32_t)std::min<size_t>(c->max_lds / (xb + 1024), (MAXW == 8 ? 8u : 12u) / W);
+        const uint32_t slots = std::max(1u, fit), cus = std::max(1u, c->cus);
+        const uint64_t wgs = (M + rows - 1) / rows, full = wgs / ((uint64_t)cus * slots);
+        const uint32_t rest = (uint32_t)((wgs - full * cus * slots + cus - 1) / cus);
+        auto round = [&](uint32_t n) {  // n workgroups on a CU
+            const uint32_t w = n * W, simd = (w + 3) / 4;
+            const float busy = simd >= 2 ? 4.0f * simd / w * (0.4f + 0.6f * w / (4.0f * simd)) : 1.4f;
+            return stage * (0.5f + 0.5f * n) + n * rows * row * busy * ((steps + S - 1) / S * S) / steps;
+        };
+        const float us = 2.0f + full * round(slots) + (rest ? round(rest) : 0.0f);
+        if (us < best.us) best = {W, S, us};
+    }
+    return best;
+}
+
 template <int F, int NC, int S, bool SILU, int DX = 0>
 void launch_gemv_s(okf_ctx *c, const GemvCall *calls, int n, uint64_t rb, uint32_t K,
-                   uint32_t cunits, size_t lds, bool pair = false) {
+                   uint32_t cunits, size_t lds, bool pair = false, uint32_t waves = 4) {
     // Q2_0 and Q8_0 at N = 1: a three-deep ring when a wavefront runs three
     // or more steps (the down projection), so that no step waits for a load
     // issued after the first compute; two otherwise (a third buffer would
     // only re-read).  Measured: Q2_0 2048x6144 4.95 -> 4.75 us.
     if constexpr (DX == 0 && NC == 1 && (F == Q2_0 || F == Q8_0)) {
         const uint32_t steps = (K / unit_weights<F>() + GV_L * S - 1) / (GV_L * S);
-        if (steps >= 3) return launch_gemv_s<F, NC, S, SILU, 3>(c, calls, n, rb, K, cunits, lds, pair);
+        if (steps >= 3) return launch_gemv_s<F, NC, S, SILU, 3>(c, calls, n, rb, K, cunits, lds, pair, waves);
     }
-    // two rows per slot (each staged activation read serves both) where
-    // measured faster: IQ2_XXS with 1..5 columns (16.9 -> 16.4 us at one), the
-    // generic formats with 2..5 (17408 x 5120, N = 4: 15-18 % faster; at one
-    // column 10-25 % slower), Q4_K and Q2_0 with 5.  (A
-    // three-deep ring for the Q4_K matvec measured 3-4 % slower than two
-    // once the weight loads were issued behind the staging's.)
-    constexpr int R = ((F == IQ2_XXS && NC >= 1) || (grid_fmt(F) && NC >= 2) ||
-                       (NC == 5 && F != Q8_0 && F != Q5_K && F != Q6_K && F != IQ4_XS)) ? 2 : 1,
-                  D = DX ? DX : 2, WAVES = 4;
+    constexpr int R = gemv_rows<F, NC>(), D = DX ? DX : 2;
     const void *fn = (const void *)gemv_kernel<F, NC, R, D, S, SILU>;
     static std::atomic<uint64_t> attr{0};  // devices that have the attribute set
     set_lds_attr(c, fn, attr);
-    const uint32_t rows_per_wg = (WAVES / S) * GV_SLOTS * R;
+    const uint32_t rows_per_wg = (waves / S) * GV_SLOTS * R;
     GemvGroup g{};
     uint32_t total = 0;
     for (int i = 0; i < n; i++) {
@@ -217,15 +271,10 @@ void launch_gemv_s(okf_ctx *c, const GemvCall *calls, int n, uint64_t rb, uint32
     // the tables the compute reads: IQ2_XXS's LDS rows (copied from c->tab),
     // or the grid formats' device-memory grids
     const u32x4 *tabs = itab_rows(F) ? c->tab8 + itab_at(F) : grid_fmt(F) ? (const u32x4 *)(c->grids + gt_off(F)) : c->tab8;
-    hipLaunchKernelGGL((gemv_kernel<F, NC, R, D, S, SILU>), dim3(total), dim3(64 * WAVES), lds, c->stream,
+    hipLaunchKernelGGL((gemv_kernel<F, NC, R, D, S, SILU>), dim3(total), dim3(64 * waves), lds, c->stream,
                        g, rb, K, tabs, cunits);
 }
 
-// Launch geometry: 256-thread workgroups of four wavefronts, each four row
-// slots of 16 lanes.  For one column with fewer than ~3072 wavefronts' worth
-// of rows, K is split two ways across the wavefronts of a workgroup (more,
-// shorter wavefronts); measured on MI355X, a four-way split loses to the
-// extra activation staging it needs.
 template <int F, int NC, uint32_t SP>
 void launch_wide_sp(okf_ctx *c, const GemvCall &call, uint64_t rb, uint32_t K, uint32_t G, size_t lds,
                     uint32_t kmax) {
@@ -460,6 +509,11 @@ bool launch_gemv_sb(okf_ctx *c, const GemvCall *calls, int n, uint64_t rb, uint3
     }
 }
 
+// Launch geometry: for one column 256-thread workgroups of four wavefronts,
+// each four row slots of 16 lanes; with fewer than ~3072 wavefronts' worth of
+// rows, K is split two ways across the wavefronts of a workgroup (more, shorter
+// wavefronts; a four-way split loses to the extra activation staging it
+// needs).  For more columns as plan_gemv says.
 template <int F, int NC, bool SILU = false>
 void launch_gemv_nc(okf_ctx *c, const GemvCall *calls, int n, uint64_t rb, uint32_t K) {
     if (launch_gemv_sb<F, NC, SILU>(c, calls, n, rb, K)) return;
@@ -476,18 +530,34 @@ void launch_gemv_nc(okf_ctx *c, const GemvCall *calls, int n, uint64_t rb, uint3
     // stage all of x when it fits, else in chunks of 64-unit groups (per
     // 32 weights: three 32-byte digit planes and a float4 of group data)
     const size_t per_unit = (size_t)NC * unit_lds_bytes<F>();
-    const size_t red = 4 * GV_SLOTS * NC * 4 * sizeof(float);
+    uint32_t rows = 0, waves = 4, S = 1;
+    for (int i = 0; i < n; i++) rows += calls[i].M;
+    if constexpr (NC > 1) {
+        const GemvPlan p = plan_gemv<F, NC>(c, rows, K);
+        if constexpr (NC >= 4 && gemv_max_waves<F, NC>() == 4) {
+            // two launches of fewer columns, on more wavefronts (Q4_K
+            // 5120 x 17408, N = 4: 63.7 -> 40.6 us)
+            if (n == 1 && plan_gemv<F, 2>(c, rows, K).us + plan_gemv<F, NC - 2>(c, rows, K).us < p.us) {
+                GemvCall call = calls[0];
+                launch_gemv_nc<F, 2, SILU>(c, &call, 1, rb, K);
+                call.X += 2 * (uint64_t)K;
+                call.Y += 2 * (uint64_t)call.M;
+                return launch_gemv_nc<F, NC - 2, SILU>(c, &call, 1, rb, K);
+            }
+        }
+        waves = p.W;
+        S = p.S;
+    }
+    const size_t red = waves * GV_SLOTS * NC * 4 * sizeof(float);
     uint32_t cunits = (units + 63) / 64 * 64;
     const size_t budget = c->max_lds - tab - red;
     if (cunits * per_unit > budget) cunits = (uint32_t)(budget / per_unit) / 64 * 64;
     const size_t lds = tab + cunits * per_unit + red;
-    uint32_t rows = 0;
-    for (int i = 0; i < n; i++) rows += calls[i].M;
     const uint32_t waves1 = (rows + GV_SLOTS - 1) / GV_SLOTS;  // wavefronts without a split
-    uint32_t S = c->gemv_s ? (uint32_t)c->gemv_s : (NC == 1 && waves1 < 3072 ? 2 : 1);
-    if (S >= 4) launch_gemv_s<F, NC, 4, SILU>(c, calls, n, rb, K, cunits, lds);
-    else if (S == 2) launch_gemv_s<F, NC, 2, SILU>(c, calls, n, rb, K, cunits, lds);
-    else launch_gemv_s<F, NC, 1, SILU>(c, calls, n, rb, K, cunits, lds);
+    if (NC == 1) S = c->gemv_s ? (uint32_t)c->gemv_s : waves1 < 3072 ? 2 : 1;
+    if (S >= 4) launch_gemv_s<F, NC, 4, SILU>(c, calls, n, rb, K, cunits, lds, false, waves);
+    else if (S == 2) launch_gemv_s<F, NC, 2, SILU>(c, calls, n, rb, K, cunits, lds, false, waves);
+    else launch_gemv_s<F, NC, 1, SILU>(c, calls, n, rb, K, cunits, lds, false, waves);
 }
 
 // Q2_0 matvecs of the Bonsai shapes on the integer matrix cores

@@ -1117,3 +1117,31 @@ def test_gemv_superblock_edges(enc_sb, t, M, K):
         assert rel(o, r.astype(np.float64)) <= TOL_MV
     for o, r in zip(*outs):
         assert rel(o, r.astype(np.float64)) <= 1e-5
+
+
+# ------------------------------------------------------------------ gemv_kernel, 2..5 columns
+# Workgroups of 4 to 12 wavefronts, K split over 1, 2 or 4 of them (forced by
+# OKF_GEMV_S; None: the planned one): one row, rows that fill no workgroup, fewer
+# steps than parts, x staged in chunks (K = 17408), Q4_K / Q5_K columns in two
+# launches.  Against the oracle at the matvec gate.
+@pytest.fixture(scope="module", params=[None, "1", "2", "4"], ids=lambda v: f"split{v or '_planned'}")
+def enc_gemv_s(request):
+    import os
+    if request.param:
+        os.environ["OKF_GEMV_S"] = request.param
+    try:
+        e = ok.Enc(0)
+    finally:
+        os.environ.pop("OKF_GEMV_S", None)
+    yield e
+    e.close()
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K, Q3_K, Q8_0, Q2_0, IQ3_XXS, F32, F16], ids=lambda t: NAMES[t])
+@pytest.mark.parametrize("M,K", [(1, 256), (2003, 768), (1025, 2304), (37, 9216), (261, 17408)])
+def test_gemv_columns_workgroups(enc_gemv_s, t, M, K):
+    say("columns", NAMES[t], M, K)
+    w, X = weights(t, M, K, 31), acts(5, K, 32)
+    ref = oracle.matmul(t, w, K, M, X).astype(np.float64)
+    for N in (2, 3, 4, 5):
+        assert rel(run_gemm(enc_gemv_s, t, M, K, w, X[:N]), ref[:N]) <= TOL_MV
