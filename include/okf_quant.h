@@ -102,10 +102,11 @@ int okf_ctx_stream(okf_ctx *ctx, void **stream);
  * okf_argmax_rows over up to argmax_rows rows of argmax_n values.  Afterwards
  * no call allocates or synchronises; one that needs more scratch than
  * reserved returns OKF_E_SHAPE.  Nor does any call allocate while the
- * context's stream is being captured into a graph.  (The tile GEMM of the other formats uses
- * the same scratch for its K-split partials and fp16 activations where it
- * fits, and otherwise runs without them: one K range, or the activations
- * rounded per tile; the K split changes only the order of the fp32 sums.)
+ * context's stream is being captured into a graph.  (The tile GEMM of the
+ * other formats uses the same scratch for its fp16 activations, and every
+ * tile GEMM for its K-split partials, where they fit, and otherwise runs
+ * without them: the activations rounded per tile, or one K range; the K
+ * split changes only the order of the fp32 sums.)
  * Without it the scratch grows on demand (hipMalloc after draining the
  * stream). */
 int okf_ctx_reserve(okf_ctx *ctx, uint64_t gemm_nk, uint32_t argmax_n, uint32_t argmax_rows);
@@ -163,9 +164,9 @@ int okf_silu_mul(okf_ctx *ctx, float *a, const float *b, uint32_t n);
 /* MetalEnc.gemm (MetalEnc.swift:241-289): Y[N][M] = X[N][K] W^T.  Dispatch
  * policy as the reference: N == 1 -> gemv; 2 <= N <= 5 -> narrow (one weight
  * pass serving all N columns, gemmNarrow / gemmNarrowIQ :176-239);
- * N > 5 -> MFMA tile GEMM (gemmTiled / iqGemmTiled, :354-400; a grid of
- * fewer than two tiles a CU splits K over workgroups, partials added in K
- * order), except that a small N past 5 (up to a per-format bound, 5..16
+ * N > 5 -> MFMA tile GEMM (gemmTiled / iqGemmTiled, :354-400; where the
+ * tiles do not fill the CUs K may be split over workgroups, partials added in
+ * K order), except that a small N past 5 (up to a per-format bound, 5..16
  * columns, where measured faster than the tile) runs as consecutive narrow
  * launches of 4 or 5 columns (for IQ2_XXS, and for every other K-quant and
  * i-quant format but Q6_K and IQ4_NL with K <= 6144 and M >= 4096, from N =
