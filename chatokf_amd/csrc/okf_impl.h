@@ -64,8 +64,10 @@ struct okf_ctx {
     int last_hip = 0;
     _Float16 *xh = nullptr;  // fp16 copy of the GEMM activations (grown on demand)
     size_t xh_bytes = 0;
-    bool captured = false;          // a captured graph holds scratch addresses: replaced buffers are
-    std::vector<void *> retired;    // kept here until the context is destroyed
+    // a captured graph holds the buffer's address: when it is replaced the old one is kept
+    // in retired until the context is destroyed (grow_buf)
+    bool xh_held = false, part_held = false, cnt_held = false;
+    std::vector<void *> retired;
     // okf_parallel_begin .. okf_parallel_end: recorded matvecs
     struct Pending {
         int32_t type;
@@ -659,55 +661,65 @@ inline bool can_grow(okf_ctx *c) {
 // Grows one scratch buffer to at least `need` bytes (the stream is drained
 // before an old buffer is freed).  Where it may not grow (can_grow) a call
 // that needs more is an OKF_E_SHAPE, so nothing on a reserved or captured
-// hot path allocates or synchronises.  `optional`: a failure leaves the
-// buffer as it was and records no HIP error (the caller runs without it).
-inline int grow_buf(okf_ctx *c, void **buf, size_t &bytes, size_t need, bool zero, bool optional) {
+// hot path allocates or synchronises.  A buffer that a captured graph holds
+// (held) is not freed but kept until the context is destroyed, and its
+// successor takes at least twice its bytes, so that the kept ones together
+// are never more than the one in use.  `optional`: a failure records no HIP
+// error (the caller runs without the buffer).
+inline int grow_buf(okf_ctx *c, void **buf, size_t &bytes, bool &held, size_t need, bool zero, bool optional) {
     if (need <= bytes) return OKF_OK;
     if (!can_grow(c)) return OKF_E_SHAPE;
     hipError_t e = hipSuccess;
+    size_t take = need;
     if (*buf) {
         e = hipStreamSynchronize(c->stream);
         if (e != hipSuccess) return optional ? ((void)hipGetLastError(), OKF_E_HIP) : hip_fail(c, e);
-        bool keep = false;
-        if (c->captured) {
+        if (held) {
             try {
                 c->retired.push_back(*buf);
-                keep = true;
             } catch (const std::bad_alloc &) {
                 return OKF_E_ARG;  // (the buffer stays as it is)
             }
+            take = std::max(need, 2 * bytes);
+        } else {
+            (void)hipFree(*buf);
         }
-        if (!keep) (void)hipFree(*buf);
         *buf = nullptr;
         bytes = 0;
+        held = false;
     }
-    e = hipMalloc(buf, need);
-    if (e == hipSuccess && zero) e = hipMemset(*buf, 0, need);
+    e = hipMalloc(buf, take);
+    if (e != hipSuccess && take > need) {
+        (void)hipGetLastError();
+        take = need;
+        e = hipMalloc(buf, take);
+    }
+    if (e == hipSuccess && zero) e = hipMemset(*buf, 0, take);
     if (e != hipSuccess) {
         if (*buf) (void)hipFree(*buf);
         *buf = nullptr;
         return optional ? ((void)hipGetLastError(), OKF_E_HIP) : hip_fail(c, e);
     }
-    bytes = need;
+    bytes = take;
     return OKF_OK;
 }
 
 // split-tile partial sums and argmax pairs
 inline int grow_part(okf_ctx *c, size_t need, bool optional = false) {
-    return grow_buf(c, (void **)&c->part, c->part_bytes, need, false, optional);
+    return grow_buf(c, (void **)&c->part, c->part_bytes, c->part_held, need, false, optional);
 }
 
 // argmax row counters, zeroed when allocated (the kernel leaves them zero)
 inline int grow_cnt(okf_ctx *c, size_t rows) {
     size_t bytes = c->cnt_n * sizeof(uint32_t);
-    const int st = grow_buf(c, (void **)&c->cnt, bytes, rows * sizeof(uint32_t), true, false);
+    const int st = grow_buf(c, (void **)&c->cnt, bytes, c->cnt_held, rows * sizeof(uint32_t), true, false);
     c->cnt_n = bytes / sizeof(uint32_t);
     return st;
 }
 
 // the fp16 copy of a GEMM's activations: N K values
 inline int grow_xh(okf_ctx *c, size_t need, bool optional = false) {
-    return grow_buf(c, (void **)&c->xh, c->xh_bytes, need, false, optional);
+    return grow_buf(c, (void **)&c->xh, c->xh_bytes, c->xh_held, need, false, optional);
 }
 
 // ---------------------------------------------------------- tile GEMM plan
@@ -786,13 +798,17 @@ inline MmPlan plan_mm(const okf_ctx *c, int type, uint32_t K, uint32_t M, uint32
     return p;  // (OKF_GEMM_PLAN is checked against the instances when it is read)
 }
 
-// Marks that a graph being captured now holds the context's scratch
-// addresses: a later growth keeps the old buffer until the context is
-// destroyed.
-inline void note_capture(okf_ctx *c) {
+// Marks the scratch buffers that a call hands to its launches, where they are
+// being captured into a graph: the graph holds their addresses (grow_buf).
+inline void note_capture(okf_ctx *c, bool xh, bool part, bool cnt) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(c->stream, &cs) != hipSuccess) (void)hipGetLastError();
-    else if (cs != hipStreamCaptureStatusNone) c->captured = true;
+    if (hipStreamIsCapturing(c->stream, &cs) != hipSuccess) {
+        (void)hipGetLastError();
+    } else if (cs != hipStreamCaptureStatusNone) {
+        c->xh_held |= xh;
+        c->part_held |= part;
+        c->cnt_held |= cnt;
+    }
 }
 
 template <int F>
@@ -824,7 +840,7 @@ int launch_gemm(okf_ctx *c, const uint8_t *W, uint64_t rb, uint32_t K, uint32_t 
         if (grow_part(c, (size_t)ks * N * M * sizeof(float), true) == OKF_OK) part = c->part;
         else ks = 1, kper = (K + MC_BK - 1) / MC_BK * MC_BK;
     }
-    note_capture(c);
+    note_capture(c, !st, part != nullptr, false);
     const u32x4 *tab = dq_tab_rows<F>() ? c->tab8 : nullptr;
     if (st) {
         dim3 grid((N + GB_N - 1) / GB_N, (M + GB_M - 1) / GB_M, ks);

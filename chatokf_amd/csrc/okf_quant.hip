@@ -577,7 +577,7 @@ int okf_argmax_rows(okf_ctx *c, const float *x, uint32_t n, uint32_t rows, int32
     const uint32_t chunks = (n + ARGMAX_CHUNK - 1) / ARGMAX_CHUNK;
     if ((st = grow_part(c, (size_t)chunks * rows * sizeof(ArgPair)))) return st;
     if ((st = grow_cnt(c, rows))) return st;
-    note_capture(c);
+    note_capture(c, false, true, true);
     hipLaunchKernelGGL(argmax_kernel, dim3(chunks, rows), dim3(NORM_THREADS), 0, c->stream, x, n,
                        (ArgPair *)c->part, c->cnt, out);
     return finish(c);

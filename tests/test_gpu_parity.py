@@ -662,6 +662,56 @@ def test_tile_gemm_graph_capture_unreserved(t, M, K, N):
         e.close()
 
 
+# A graph captured after an eager call holds the scratch (the fp16 X, the K
+# ranges' partial sums that are the argmax's pairs too, the row counters);
+# larger eager calls then replace it, and replays between and after them must
+# still give the eager bits.
+def test_graph_keeps_its_scratch_over_growth():
+    hip = ctypes.CDLL("libamdhip64.so")
+    vp = ctypes.c_void_p
+    e = ok.Enc(0)
+    try:
+        M, K, N = 512, 2048, 40
+        qw = ok.QuantTensor(dev(weights(Q4_K, M, K, 96)), K, M, Q4_K)
+        Xd = dev(acts(N, K, 97))
+        Y, top = torch.zeros((N, M), device="cuda"), torch.zeros(N, dtype=torch.int32, device="cuda")
+
+        def work():
+            e.gemm(qw, Xd, Y, N)
+            e.argmax_rows(Y, M, N, top)
+
+        work()
+        e.sync()
+        want = host(Y), host(top)
+        st = vp(e.stream)
+        graph, exe = vp(), vp()
+        assert hip.hipStreamBeginCapture(st, 0) == 0
+        work()
+        assert hip.hipStreamEndCapture(st, ctypes.byref(graph)) == 0
+        assert hip.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, 0) == 0
+        try:
+            for n in (N, 300, 700):
+                say("graph over growth", n)
+                Xl, Yl = dev(acts(n, K, 98)), torch.zeros((n, M), device="cuda")
+                tl = torch.zeros(n, dtype=torch.int32, device="cuda")
+                e.gemm(qw, Xl, Yl, n)  # (n > N: grows all three)
+                e.argmax_rows(Yl, M, n, tl)
+                e.sync()
+                for _ in range(2):
+                    Y.fill_(float("nan"))
+                    top.fill_(-1)
+                    torch.cuda.synchronize()
+                    assert hip.hipGraphLaunch(exe, st) == 0
+                    assert hip.hipStreamSynchronize(st) == 0
+                    assert np.array_equal(host(Y), want[0]) and np.array_equal(host(top), want[1])
+                assert np.array_equal(host(tl), oracle.argmax_rows(host(Yl)))
+        finally:
+            hip.hipGraphExecDestroy(exe)
+            hip.hipGraphDestroy(graph)
+    finally:
+        e.close()
+
+
 # The grid barrier's bounded wait, forced from the host: OKF_FFN_STALL=1
 # makes the next launch's barrier wait for one arrival more than the grid
 # has, OKF_FFN_SPIN a short poll limit.  Every workgroup still finishes; the

@@ -28,3 +28,28 @@ def test_captured_argmax_keeps_its_scratch(fake, grow):
     assert len(held) == 2 and len(r[3]["allocs"]) == len(r[1]["allocs"])  # pairs, counters; nothing in the capture
     assert len(r[-1]["allocs"]) > len(r[1]["allocs"])                     # (it did grow)
     assert [r[-1]["allocs"][i][1] for i in held] == [0, 0]
+
+
+# What is kept is bounded: a buffer that no graph holds is freed when it is
+# replaced, and one that a graph holds by a successor of at least twice its size.
+def test_kept_scratch_is_bounded(fake):
+    steps = [["norm", 64, 1, 0], ["argmax", 248320, 1], ["capture", 1], ["argmax", 248320, 1], ["capture", 0]]
+    for rows in range(2, 70):
+        steps.append(["argmax", 248320, rows])
+        if rows < 20:  # (a graph after each growth, then growth without graphs)
+            steps += [["capture", 1], ["argmax", 248320, rows], ["capture", 0]]
+    r = fakehip.run(fake, steps)
+    base = len(r[0]["allocs"])
+    for s in r:
+        live = [n for n, freed in s["allocs"][base:] if not freed]
+        pairs = sorted(n for n in live if n >= 122 * 8)
+        assert sum(pairs[:-1]) <= (pairs[-1] if pairs else 0)
+    assert sum(f for n, f in r[-1]["allocs"][base:]) > 0
+
+
+# The buffers that a capture did not hand to a launch are not held by it.
+def test_capture_holds_what_it_uses(fake):
+    r = fakehip.run(fake, [["gemm", "q4_k", 5120, 17408, 64], ["argmax", 1000, 1], ["capture", 1], ["argmax", 1000, 1],
+                           ["capture", 0], ["gemm", "q4_k", 5120, 17408, 128]])
+    xh = 64 * 17408 * 2
+    assert [f for n, f in r[-1]["allocs"] if n == xh] == [1]
