@@ -755,7 +755,10 @@ inline bool mm_instance(int kind, int fm, int fn) {
 //  K ranges: the partial tiles written and read at 5 TB/s, and a launch.
 // From 256 tokens on the formats but Q4_K take only many, whose sums are in
 // gemm_mfma_kernel's order (few takes K in another order within 128).
-inline MmPlan plan_mm(const okf_ctx *c, int type, uint32_t K, uint32_t M, uint32_t N) {
+// room: bytes there are for partial tiles; a plan takes as many K ranges as fit
+// (without room for two, one range, whose best tile is another: Q4_K 5120 x
+// 17408, N = 64, 64 workgroups of the K-split plan's tile 113 us, the one-range plan 56).
+inline MmPlan plan_mm(const okf_ctx *c, int type, uint32_t K, uint32_t M, uint32_t N, size_t room = SIZE_MAX) {
     const uint32_t cus = c->cus ? c->cus : 256;
     auto up = [](uint64_t a, uint64_t b) { return (a + b - 1) / b; };
     MmPlan p{};
@@ -765,6 +768,7 @@ inline MmPlan plan_mm(const okf_ctx *c, int type, uint32_t K, uint32_t M, uint32
     auto consider = [&](int kind, int fm, int fn, uint32_t ks) {
         if (force[1] && (kind != force[0] || fm != force[1] || fn != force[2])) return;
         if (force[1]) ks = (uint32_t)force[3];
+        ks = (uint32_t)std::min<uint64_t>(ks, std::max<uint64_t>(1, room / ((uint64_t)N * M * sizeof(float))));
         const uint32_t unit = kind ? MC_BK : 128, steps = (uint32_t)up(K, unit);
         const uint32_t per = (uint32_t)up(steps, std::max(1u, std::min(ks, steps)));
         ks = (uint32_t)up(steps, per);
@@ -814,32 +818,33 @@ inline void note_capture(okf_ctx *c, bool xh, bool part, bool cnt) {
 template <int F>
 int launch_gemm(okf_ctx *c, const uint8_t *W, uint64_t rb, uint32_t K, uint32_t M, const float *X,
                 uint32_t N, float *Y) {
-    const MmPlan p = plan_mm(c, F, K, M, N);
     // fp16 activations, converted once per call into the context's buffer
     // (as octets: x_to_octets_kernel)
     const int st = c->gemm_xh || F == Q4_K ? grow_xh(c, (size_t)N * K * sizeof(_Float16), F != Q4_K) : OKF_E_SHAPE;
     if (st && F == Q4_K) return st;
-    uint32_t ks = p.ks, kper = p.kper;
+    // the K ranges' partial tiles, added in K order by gemm_ksum_kernel
+    auto partials = [&](uint32_t ks) { return grow_part(c, (size_t)ks * N * M * sizeof(float), true) == OKF_OK; };
+    MmPlan p = plan_mm(c, F, K, M, N);
     if (st && c->gemm_xh) {
-        // no room for them: gemm_mfma_kernel, which rounds X per tile.  A grid
+        // no room for X: gemm_mfma_kernel, which rounds X per tile.  A grid
         // of fewer than two tiles a CU (small M or N) takes K in ks ranges of
-        // whole 64-steps.
+        // whole 64-steps; without room for their partial tiles, one range.
         const uint32_t tiles = ((N + GB_N - 1) / GB_N) * ((M + GB_M - 1) / GB_M), steps = (K + GB_K - 1) / GB_K;
-        ks = 1;
+        p.ks = 1;
         if (c->gemm_split != 0 && tiles < 2 * c->cus) {
-            ks = c->gemm_split > 1 ? (uint32_t)c->gemm_split : (2 * c->cus + tiles - 1) / tiles;
-            ks = std::max(1u, std::min(ks, steps / 4));
+            p.ks = c->gemm_split > 1 ? (uint32_t)c->gemm_split : (2 * c->cus + tiles - 1) / tiles;
+            p.ks = std::max(1u, std::min(p.ks, steps / 4));
         }
-        kper = (steps + ks - 1) / ks * GB_K;
-        ks = (K + kper - 1) / kper;
+        p.kper = (steps + p.ks - 1) / p.ks * GB_K;
+        p.ks = (K + p.kper - 1) / p.kper;
+        if (p.ks > 1 && !partials(p.ks)) p.ks = 1, p.kper = steps * GB_K;
+    } else if (p.ks > 1 && !partials(p.ks)) {
+        // (a reserved context, a stream being captured, or no memory: planned
+        // again for the room that there is)
+        p = plan_mm(c, F, K, M, N, c->part_bytes);
     }
-    // the K ranges' partial tiles, added in K order by gemm_ksum_kernel;
-    // without room for them, one range
-    float *part = nullptr;
-    if (ks > 1) {
-        if (grow_part(c, (size_t)ks * N * M * sizeof(float), true) == OKF_OK) part = c->part;
-        else ks = 1, kper = (K + MC_BK - 1) / MC_BK * MC_BK;
-    }
+    const uint32_t ks = p.ks, kper = p.kper;
+    float *part = ks > 1 ? c->part : nullptr;
     note_capture(c, !st, part != nullptr, false);
     const u32x4 *tab = dq_tab_rows<F>() ? c->tab8 : nullptr;
     if (st) {

@@ -20,7 +20,7 @@ struct Alloc {
 std::map<const void *, std::string> kernels;  // host stub -> device name
 std::vector<std::string> launches;            // "name gx gy gz bx by bz lds"
 std::vector<Alloc> allocs;                    // in order; a freed one is kept, so no address comes back
-int capturing, fail_above;                    // fail_above: MiB from which hipMalloc fails (0: never)
+int capturing, fail_above;                    // fail_above: KiB from which hipMalloc fails (0: never)
 dim3 cfg_grid, cfg_block;
 size_t cfg_lds;
 hipStream_t cfg_stream;
@@ -28,7 +28,7 @@ hipStream_t cfg_stream;
 
 extern "C" {
 void fake_capture(int on) { capturing = on; }
-void fake_fail_above(int mib) { fail_above = mib; }
+void fake_fail_above(int kib) { fail_above = kib; }
 int fake_launches() { return (int)launches.size(); }
 const char *fake_launch(int i) { return launches[i].c_str(); }
 int fake_allocs() { return (int)allocs.size(); }
@@ -63,7 +63,7 @@ hipError_t hipLaunchCooperativeKernel(const void *f, dim3 g, dim3 b, void **a, u
     return hipLaunchKernel(f, g, b, a, lds, s);
 }
 hipError_t hipMalloc(void **p, size_t n) {
-    if (fail_above && n >= (size_t)fail_above << 20) return *p = nullptr, hipErrorOutOfMemory;
+    if (fail_above && n >= (size_t)fail_above << 10) return *p = nullptr, hipErrorOutOfMemory;
     *p = malloc(n);
     allocs.push_back({*p, n, false});
     return *p ? hipSuccess : hipErrorOutOfMemory;

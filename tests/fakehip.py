@@ -67,8 +67,8 @@ class _Child:
     def capture(self, on):
         self.fake.fake_capture(on)
 
-    def fail_above(self, mib):
-        self.fake.fake_fail_above(mib)
+    def fail_above(self, kib):
+        self.fake.fake_fail_above(kib)
 
     def close(self):
         self.enc.close()

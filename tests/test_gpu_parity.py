@@ -427,6 +427,24 @@ def test_reserve_then_no_allocation():
         e.close()
 
 
+# A reserved context has no room for the K ranges' partial sums, so the plan is
+# one for a single range (another tile, the same operands rounded the same):
+# against the unreserved context's split plan to fp32 sums in another order, and
+# the oracle.
+@pytest.mark.parametrize("t,M,K,N", [(Q4_K, 640, 8704, 101), (IQ4_XS, 640, 8704, 300), (Q8_0, 333, 6176, 64)])
+def test_reserved_tile_gemm_one_range(enc, t, M, K, N):
+    say("reserved tile", NAMES[t], M, K, N)
+    e = ok.Enc(0)
+    try:
+        e.reserve(N * K, 1000, 1)
+        w, X = weights(t, M, K, 44), acts(N, K, 45)
+        got = run_gemm(e, t, M, K, w, X)
+        assert rel(got, oracle.matmul(t, w, K, M, X).astype(np.float64)) <= TOL
+        assert rel(got, run_gemm(enc, t, M, K, w, X).astype(np.float64)) <= 1e-5
+    finally:
+        e.close()
+
+
 # ------------------------------------------------------------ SiLU-gated FFN
 def test_silu_mul_matches_oracle(enc):
     a = np.random.default_rng(4).standard_normal(6144).astype(np.float32) * 3

@@ -53,3 +53,40 @@ def test_capture_holds_what_it_uses(fake):
                            ["capture", 0], ["gemm", "q4_k", 5120, 17408, 128]])
     xh = 64 * 17408 * 2
     assert [f for n, f in r[-1]["allocs"] if n == xh] == [1]
+
+
+# ------------------------------------------------------------------ tile GEMM plans
+def tile_launch(step):
+    """The tile kernel of a GEMM step: (name, template arguments, workgroups, K ranges)."""
+    (k,) = [v for v in step["launches"] if v["name"] in ("gemm_few_kernel", "gemm_many_kernel", "gemm_mfma_kernel")]
+    return k["name"], k["args"], k["grid"][0] * k["grid"][1], k["grid"][2]
+
+
+# A context whose partial-sum buffer may not grow (reserved: it holds the argmax
+# pairs only; or its stream is being captured; or no memory) plans for one K
+# range: the tile that fills the CUs without a split, not the split plan's tile
+# on the fraction of the CUs that it was cut for.
+@pytest.mark.parametrize("fmt,M,K,N", [("q4_k", 5120, 17408, 64), ("q4_k", 5120, 17408, 333), ("q4_k", 2048, 6144, 101),
+                                       ("iq4_xs", 5120, 17408, 333), ("q8_0", 2048, 6144, 512), ("q2_k", 2048, 6144, 20)])
+@pytest.mark.parametrize("how", ["reserved", "captured", "memory"])
+def test_one_range_is_planned_as_one(fake, fmt, M, K, N, how):
+    call, warm = ["gemm", fmt, M, K, N], ["tile", fmt, 1 << 18, K, N]  # (warm: many rows, no split; grows X's buffer, not the partials)
+    limit = {"reserved": [["reserve", N * K, 248320, 1]], "captured": [warm, ["capture", 1]],
+             "memory": [warm, ["fail_above", 1]]}[how]
+    free = fakehip.run(fake, [call])[-1]
+    one = fakehip.run(fake, [call], OKF_GEMM_SPLIT="0")[-1]
+    got = fakehip.run(fake, limit + [call])[-1]
+    assert [s["status"] for s in (free, one, got)] == [0, 0, 0]
+    assert tile_launch(free)[3] > 1 and "gemm_ksum_kernel" in [v["name"] for v in free["launches"]]
+    assert tile_launch(got)[3] == 1 and "gemm_ksum_kernel" not in [v["name"] for v in got["launches"]]
+    assert tile_launch(got)[2] > tile_launch(free)[2]
+    if N >= 256 and fmt != "q4_k":  # (gemm_few_kernel is not planned: OKF_GEMM_SPLIT=0 plans one range of the same)
+        assert tile_launch(got) == tile_launch(one)
+
+
+# With room for some of the ranges, as many as fit.
+def test_ranges_that_fit(fake):
+    M, K, N = 5120, 17408, 64
+    r = fakehip.run(fake, [["tile", "q4_k", M, K // 17, N], ["reserve", N * K, 248320, 2 * M * N * 4 // 976 + 1],
+                           ["gemm", "q4_k", M, K, N]])
+    assert tile_launch(r[-1])[3] == 2
