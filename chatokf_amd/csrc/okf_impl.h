@@ -417,9 +417,7 @@ void launch_sb_t(okf_ctx *c, const GemvGroup &g, uint32_t total, uint64_t rb, ui
         case 1: go(std::integral_constant<int, 1>{}); break;
         case 2: go(std::integral_constant<int, 2>{}); break;
         case 3: go(std::integral_constant<int, 3>{}); break;
-        case 4:
-        case 5: go(std::integral_constant<int, 5>{}); break;
-        default: go(std::integral_constant<int, 9>{}); break;
+        default: go(std::integral_constant<int, 5>{}); break;
     }
 }
 
@@ -473,8 +471,12 @@ bool launch_gemv_sb(okf_ctx *c, const GemvCall *calls, int n, uint64_t rb, uint3
         if (F == IQ2_XXS && (lng || pair)) return false;  // (long or paired rows: gemv_kernel is no slower)
         uint32_t T = c->gemv_sb_t ? (uint32_t)c->gemv_sb_t : lng ? 512 : 256;
         if (T != 256 && T != 512) T = 256;
-        const uint32_t sr = (K / 8 + T - 1) / T;  // staging rounds
-        if (sr > 9) return false;
+        // staging rounds: at most five (K <= 20480), which the registers hold; with
+        // nine, 73 to 175 registers a lane spilled (us, gemv_kernel or
+        // gemv_wide_kernel -> nine rounds, 8192 x 28672: Q8_0 77 -> 253, Q5_K 65 ->
+        // 154, Q4_0 62 -> 110, IQ4_NL 68 -> 101, IQ4_XS 57 -> 93, Q4_K 51 -> 109)
+        const uint32_t sr = (K / 8 + T - 1) / T;
+        if (sr > 5) return false;
         uint32_t RW = c->gemv_sb_rw ? (uint32_t)c->gemv_sb_rw
                       : lng       ? std::min(32u, std::max(4u, (M + c->cus - 1) / c->cus))
                                   : std::max(1u, T / nsb) * (F == IQ2_XXS && c->gemv_sb_r == 2 ? 2 : 1);

@@ -1140,8 +1140,8 @@ def test_tile_gemm_instances(plan):
 # ------------------------------------------------------------------ superblock-per-lane matvec
 # gemv_sb_kernel, forced (OKF_GEMV_SB=1) and off (0), at its edges: one row, one
 # superblock, rows that fill no workgroup, short rows (a superblock a lane)
-# and long ones (> 32 superblocks, several a lane), single, grouped and paired
-# with the SiLU.  Against the oracle at the matvec gate, and against the
+# and long ones (> 32 superblocks, several a lane; 80, the longest, and past it),
+# single, grouped and paired with the SiLU.  Against the oracle at the matvec gate, and against the
 # general kernel to 1e-5 (both sum exact integer group products; only the
 # fp32 order of the groups differs).
 @pytest.fixture(scope="module")
@@ -1160,7 +1160,8 @@ def enc_sb():
 
 
 @pytest.mark.parametrize("t", [Q4_K, Q5_K, IQ4_XS, Q4_0, IQ4_NL, Q8_0], ids=lambda t: NAMES[t])
-@pytest.mark.parametrize("M,K", [(1, 256), (7, 768), (1001, 2304), (300, 8192), (13, 8448), (700, 10240)])
+@pytest.mark.parametrize("M,K", [(1, 256), (7, 768), (1001, 2304), (300, 8192), (13, 8448), (700, 10240), (261, 20480),
+                                 (130, 28672)])
 def test_gemv_superblock_edges(enc_sb, t, M, K):
     say("superblock matvec", NAMES[t], M, K)
     w, X = weights(t, M, K, 27), acts(1, K, 28)

@@ -90,3 +90,15 @@ def test_ranges_that_fit(fake):
     r = fakehip.run(fake, [["tile", "q4_k", M, K // 17, N], ["reserve", N * K, 248320, 2 * M * N * 4 // 976 + 1],
                            ["gemm", "q4_k", M, K, N]])
     assert tile_launch(r[-1])[3] == 2
+
+
+# ------------------------------------------------------------------ superblock matvec
+# gemv_sb_kernel keeps a lane's staged activations in registers: up to five
+# rounds (K = 20480); longer rows stay with the other matvecs, alone and paired.
+@pytest.mark.parametrize("fmt", ["q8_0", "q5_k", "q4_0", "iq4_nl", "iq4_xs", "q4_k"])
+def test_superblock_matvec_rows(fake, fmt):
+    ks = (17408, 20480, 20736, 24576, 28672, 36864)
+    r = fakehip.run(fake, [["gemv", fmt, 8192, K] for K in ks] + [["gate_up", fmt, 8192, K] for K in ks])
+    assert [s["status"] for s in r] == [0] * len(r)
+    sb = [s["launches"][0]["name"] == "gemv_sb_kernel" for s in r]
+    assert sb == 2 * [K <= 20480 for K in ks]
