@@ -1137,6 +1137,49 @@ def test_tile_gemm_instances(plan):
         e.close()
 
 
+# A block whose fp16 scale is infinite (or NaN): its weights are scale times code,
+# +-inf, and NaN for a zero code, and the sums over positive activations keep
+# that.  Row m's block 0 has scale SPECIAL[m % 4] and every other byte alike
+# (one sign a row for most), the other blocks as they were; both tile kernels,
+# against the inf / NaN pattern of the oracle's dequantized rows times X, and its
+# values where they are finite.
+SPECIAL = (np.inf, -np.inf, np.nan, 0.004)
+D_OFF = {Q8_0: 0, Q2_0: 0, Q4_0: 0, IQ4_NL: 0, Q4_K: 0, Q5_K: 0, Q6_K: 208, IQ4_XS: 0, IQ2_XXS: 0}
+
+
+@pytest.mark.parametrize("plan", ["0,1,1,1", "1,4,1,1"])
+def test_tile_gemm_infinite_scale(plan):
+    import os
+    os.environ["OKF_GEMM_PLAN"] = plan
+    try:
+        e = ok.Enc(0)
+    finally:
+        del os.environ["OKF_GEMM_PLAN"]
+    try:
+        for t, off in D_OFF.items():
+            say("infinite scale", plan, NAMES[t])
+            M, K, N = 64, 512, 20
+            bb = row_bytes(t, 256) // (8 if t in (Q8_0, Q4_0, IQ4_NL) else 2 if t == Q2_0 else 1)
+            w = weights(t, M, K, 33).copy().reshape(M, -1)
+            for m in range(M):
+                w[m, :bb] = (0, 0xFF, 0x55, 0xAA, 0x05, 0x88, 0x11, 0xF0)[m // 4 % 8]
+                if t in (Q4_K, Q5_K):
+                    w[m, 2:4] = np.array([0.004], np.float16).view(np.uint8)
+                w[m, off:off + 2] = np.array([SPECIAL[m % 4]], np.float16).view(np.uint8)
+            X = np.abs(acts(N, K, 34)) + np.float32(0.01)
+            W = np.stack([oracle.dequant(t, w[m], K) for m in range(M)]).astype(np.float64)
+            with np.errstate(invalid="ignore"):
+                ref = (X.astype(np.float64)[:, None] * W).sum(2)
+            got = run_gemm(e, t, M, K, w.reshape(-1), X, tile=True).astype(np.float64)
+            assert np.isinf(ref).any() and np.isnan(ref).any() and np.isfinite(ref).any()
+            assert np.array_equal(np.isnan(got), np.isnan(ref))
+            assert np.array_equal(np.where(np.isinf(got), got, 0), np.where(np.isinf(ref), ref, 0))
+            fin = np.isfinite(ref)
+            assert np.abs(got[fin] - ref[fin]).max() <= TOL * np.abs(ref[fin]).max()
+    finally:
+        e.close()
+
+
 # ------------------------------------------------------------------ superblock-per-lane matvec
 # gemv_sb_kernel, forced (OKF_GEMV_SB=1) and off (0), at its edges: one row, one
 # superblock, rows that fill no workgroup, short rows (a superblock a lane)
