@@ -770,6 +770,7 @@ inline MmPlan plan_mm(const okf_ctx *c, int type, uint32_t K, uint32_t M, uint32
     auto consider = [&](int kind, int fm, int fn, uint32_t ks) {
         if (force[1] && (kind != force[0] || fm != force[1] || fn != force[2])) return;
         if (force[1]) ks = (uint32_t)force[3];
+        if (!kind && up(N, 16 * fn) > 65535) return;  // (the grid's second dimension; many has all tiles in the first)
         ks = (uint32_t)std::min<uint64_t>(ks, std::max<uint64_t>(1, room / ((uint64_t)N * M * sizeof(float))));
         const uint32_t unit = kind ? MC_BK : 128, steps = (uint32_t)up(K, unit);
         const uint32_t per = (uint32_t)up(steps, std::max(1u, std::min(ks, steps)));

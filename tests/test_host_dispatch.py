@@ -92,6 +92,15 @@ def test_ranges_that_fit(fake):
     assert tile_launch(r[-1])[3] == 2
 
 
+# Millions of tokens on a few rows: within the grid's limits (65535 in y and z).
+@pytest.mark.parametrize("M,K,N", [(1, 512, 4200001), (16, 512, 4200001), (64, 256, 2000000)])
+def test_many_tokens_fit_the_grid(fake, M, K, N):
+    (r,) = fakehip.run(fake, [["gemm", "q4_k", M, K, N]])
+    assert r["status"] == 0
+    for v in r["launches"]:
+        assert max(v["grid"][1:]) <= 65535 and v["grid"][0] * v["block"] < 1 << 32
+
+
 # ------------------------------------------------------------------ superblock matvec
 # gemv_sb_kernel keeps a lane's staged activations in registers: up to five
 # rounds (K = 20480); longer rows stay with the other matvecs, alone and paired.
