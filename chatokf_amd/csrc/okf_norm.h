@@ -33,10 +33,13 @@ __device__ __forceinline__ float block_sum(float v, float *red) {
 // before the first is used, so that nothing is loaded behind the sum.  NT =
 // 1024 where there are fewer rows than CUs (a decode step's one row: a thread
 // waits for one or two loads instead of five): 1 x 5120 3.6 -> 2.6 us, with r
-// 3.8 -> 3.0, 64 x 5120 3.9 -> 2.9.  More rows without r: NT = 512, 512 x 5120 6.2
-// -> 5.2; with r they stream 84 KB a row from memory, and fewer registers a
-// wavefront is what counts: NT = 256, not ahead (1024 x 5120 12.9 us; NT = 512
-// ahead 14.4).
+// 3.8 -> 3.0, 64 x 5120 3.9 -> 2.9.  More rows without r, of more than 1024
+// values: NT = 512 ahead (512 x 5120 5.4 -> 4.9, 512 x 2048 3.6 -> 3.3); past
+// four rows a CU only of more than 2048 (1024 x 5120 7.9 -> 7.2, but 2000 x 2048
+// 6.4 -> 6.6).  Short rows leave most of 512 threads idle: NT = 256, not ahead
+// (16384 x 128 14.7 us, NT = 512 ahead 25.1; 2000 x 1024 4.7 against 5.9), and so
+// all rows with r, which stream 84 KB a row of 5120 from memory, where fewer
+// registers a wavefront is what counts (1024 x 5120 13.0 us; NT = 512 ahead 14.6).
 template <bool ADD, int NT, bool AHEAD>
 __global__ __launch_bounds__(NT) void add_rmsnorm_kernel(float *X, const float *__restrict__ R,
                                                          const float *__restrict__ Wn, float *Y, uint32_t n,

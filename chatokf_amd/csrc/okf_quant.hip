@@ -564,8 +564,10 @@ int okf_add_rmsnorm_batch(okf_ctx *c, float *x, const float *r, const float *w, 
         hipLaunchKernelGGL(kern, dim3(rows), dim3(nt), 0, c->stream, x, r, w, y, n, eps);
     };
     const bool few = rows < c->cus;  // (fewer rows than CUs: more threads a row)
+    const bool wide = n > 2048 || (n > 1024 && rows < 4 * c->cus);
     if (r) few ? go(add_rmsnorm_kernel<true, 1024, true>, 1024) : go(add_rmsnorm_kernel<true, 256, false>, 256);
-    else few ? go(add_rmsnorm_kernel<false, 1024, true>, 1024) : go(add_rmsnorm_kernel<false, 512, true>, 512);
+    else if (few) go(add_rmsnorm_kernel<false, 1024, true>, 1024);
+    else wide ? go(add_rmsnorm_kernel<false, 512, true>, 512) : go(add_rmsnorm_kernel<false, 256, false>, 256);
     return finish(c);
 }
 

@@ -315,8 +315,10 @@ def test_wide_matches_oracle_and_default(enc, enc_wide, t, M, K, N):
 
 # ---------------------------------------------- add + RMSNorm, argmax
 # n: vector path (multiple of 4, <= 8192), scalar paths (odd n, n > 8192, a
-# pointer off 16-byte alignment); rows as decode (1) and MTP verify (5)
-NORM = [(2048, 1, 0), (5120, 5, 0), (6144, 3, 0), (10000, 2, 0), (1001, 3, 0), (2048, 2, 1)]
+# pointer off 16-byte alignment); rows as decode (1) and MTP verify (5), and
+# past one and four a CU of 256 (other workgroups: okf_add_rmsnorm_batch)
+NORM = [(2048, 1, 0), (5120, 5, 0), (6144, 3, 0), (10000, 2, 0), (1001, 3, 0), (2048, 2, 1), (128, 1500, 0),
+        (1028, 300, 0), (2052, 1100, 0), (1001, 300, 0), (2048, 300, 1), (10000, 260, 0)]
 
 
 @pytest.mark.parametrize("n,rows,skew", NORM)

@@ -111,3 +111,15 @@ def test_superblock_matvec_rows(fake, fmt):
     assert [s["status"] for s in r] == [0] * len(r)
     sb = [s["launches"][0]["name"] == "gemv_sb_kernel" for s in r]
     assert sb == 2 * [K <= 20480 for K in ks]
+
+
+# ------------------------------------------------------------------ RMSNorm
+# Threads a row: short rows past one a CU keep 256 (a head's norm over 128
+# values took 25.1 us for 16384 rows on 512 threads, 14.7 on 256).
+@pytest.mark.parametrize("n,rows,add,threads", [(128, 16384, 0, 256), (1024, 300, 0, 256), (1536, 300, 0, 512),
+                                                (2048, 1023, 0, 512), (2048, 1024, 0, 256), (2052, 2000, 0, 512),
+                                                (5120, 512, 1, 256), (5120, 255, 0, 1024), (128, 1, 1, 1024)])
+def test_norm_threads(fake, n, rows, add, threads):
+    (r,) = fakehip.run(fake, [["norm", n, rows, add]])
+    (v,) = r["launches"]
+    assert (v["block"], v["grid"]) == (threads, [rows, 1, 1]) and v["args"][:2] == [add, threads]
