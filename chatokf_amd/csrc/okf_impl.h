@@ -431,7 +431,8 @@ void launch_sb_t(okf_ctx *c, const GemvGroup &g, uint32_t total, uint64_t rb, ui
 // 3584 (172 K) 7.2 -> 7.7, 17408 x 5120 12.4 -> 11.5, 5120 x 17408 19.9 -> 13.5;
 // IQ4_NL 17408 x 5120 (348 K) 14.9 -> 15.3, 60000 x 2048 18.7 -> 17.0, 5120 x 17408
 // 22.0 -> 17.2; IQ2_XXS 2048 x 2048 4.1 -> 7.6, 12288 x 3584 9.8 -> 11.4, 17408 x 5120
-// 14.9 -> 13.9, 60000 x 2048 15.6 -> 16.6.  Gate and up paired (okf_ffn, H x D):
+// 14.9 -> 13.9, 60000 x 2048 16.2 -> 17.6, 120000 x 1536 25.0 -> 22.0, 248320 x 1024
+// 33.0 -> 26.6, 248320 x 4096 89.5 -> 83.1, 60000 x 512 10.6 -> 8.9.  Gate and up paired (okf_ffn, H x D):
 // 6144 x 2048 Q4_K 10.6 -> 10.8, Q5_K 11.6 -> 11.9, Q8_0 12.5 -> 13.1; 7168 x 3584 Q4_K
 // 16.4 -> 16.0, Q5_K 20.7 -> 17.7, IQ4_NL 18.3 -> 19.7; 17408 x 5120 Q4_K 37.2 -> 35.8,
 // Q5_K 55.6 -> 41.9, IQ4_XS 50.6 -> 44.9, IQ4_NL 55.6 -> 45.3, Q4_0 52.6 -> 35.7, Q8_0
@@ -444,7 +445,7 @@ bool sb_auto(uint64_t rows, uint32_t K, bool pair) {
     switch (F) {
         case Q4_K: return lng || n >= 30000;
         case Q5_K: return n >= 30000;
-        case IQ2_XXS: return n >= 100000 && K >= 5120;
+        case IQ2_XXS: return (n >= 100000 && K >= 5120) || rows >= 120000 || (K <= 512 && rows >= 50000);
         case Q4_0: return n >= (lng ? 96000u : 300000u);
         case IQ4_NL: return n >= (lng ? 96000u : 400000u);
         default: return n >= 96000;  // Q8_0, IQ4_XS

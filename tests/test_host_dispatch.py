@@ -113,6 +113,14 @@ def test_superblock_matvec_rows(fake, fmt):
     assert sb == 2 * [K <= 20480 for K in ks]
 
 
+# IQ2_XXS: tall matrices of short rows too (248320 x 1024 33.0 us on gemv_kernel, 26.6).
+@pytest.mark.parametrize("M,K,sb", [(248320, 1024, True), (120000, 2048, True), (60000, 512, True), (60000, 2048, False),
+                                    (6144, 2048, False), (17408, 5120, True), (30000, 256, False)])
+def test_superblock_matvec_iq2_xxs(fake, M, K, sb):
+    (r,) = fakehip.run(fake, [["gemv", "iq2_xxs", M, K]])
+    assert [v["name"] for v in r["launches"]] == ["gemv_sb_kernel" if sb else "gemv_kernel"]
+
+
 # ------------------------------------------------------------------ RMSNorm
 # Threads a row: short rows past one a CU keep 256 (a head's norm over 128
 # values took 25.1 us for 16384 rows on 512 threads, 14.7 on 256).
