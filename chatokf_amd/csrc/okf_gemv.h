@@ -1433,8 +1433,10 @@ struct GemvGroup {
 // Wavefronts a workgroup of gemv_kernel may have: four for one column.  With
 // more columns the staged x leaves room for one workgroup of long rows per CU,
 // and four wavefronts are too few to hide the LDS reads of one another: twelve
-// where the kernel's registers allow (168 each), else eight (256).  Q4_K and
-// Q5_K with four and five columns take all 512 and stay at four.
+// where the kernel does with 168 registers (one to seven spilled in a few, which costs
+// less than fewer wavefronts: Q6_K, N = 3 / 4, 17408 x 5120 31.2 / 36.7 us, with
+// eight 37.6 / 45.5), else eight (256).  Q4_K and Q5_K with four and five
+// columns take all 512 and stay at four.
 template <int F, int NC>
 __host__ __device__ constexpr uint32_t gemv_max_waves() {
     if (NC == 1) return 4;
@@ -1445,11 +1447,13 @@ __host__ __device__ constexpr uint32_t gemv_max_waves() {
     return 12;
 }
 
-template <int F, int NC, int R, int D, int S, bool SILU>
-__global__ __launch_bounds__((64 * gemv_max_waves<F, NC>())) void gemv_kernel(GemvGroup g, uint64_t row_bytes,
-                                                                              uint32_t K,
-                                                                              const u32x4 *__restrict__ tab_g,
-                                                                              uint32_t cunits) {
+// MW: the most wavefronts a workgroup of this instance has.  (Four-wavefront
+// calls of several columns have an instance of their own: within the registers of
+// twelve F32, N = 2, took 522 us at 151936 x 2048 against 438, Q8_0 55.9 against
+// 52.2 at 248320 x 1024.)
+template <int F, int NC, int R, int D, int S, bool SILU, uint32_t MW>
+__global__ __launch_bounds__(64 * MW) void gemv_kernel(GemvGroup g, uint64_t row_bytes, uint32_t K,
+                                                       const u32x4 *__restrict__ tab_g, uint32_t cunits) {
     uint32_t i = 0;
 #pragma unroll
     for (int k = 0; k + 1 < GV_GROUP; k++)

@@ -214,16 +214,30 @@ GemvPlan plan_gemv(const okf_ctx *c, uint64_t M, uint32_t K) {
     const size_t xb = (size_t)NC * K / unit_weights<F>() * unit_lds_bytes<F>() + gemv_tab_rows<F>() * 16;
     const float k = K / 14336.0f, stage = 0.5f + k * (2.3f + 2.05f * NC), row = k * (0.17f + 0.13f * NC);
     GemvPlan best{4, 1, 1e30f};
-    // (many short rows: small workgroups, several on a CU, stage while others
-    // compute; Q8_0 N = 2 at 30000 x 2048 14.4 us, with larger ones 17.9; at
-    // 20000 x 4096 17.5 against 18.9)
-    const bool many = !c->gemv_s && K <= 4096 && M > 64ull * c->cus;
+    // Many short rows take four wavefronts and no split: small workgroups, several
+    // on a CU (the four-wavefront instance of these formats does with few enough
+    // registers for 12 to 24 wavefronts), stage while others compute; Q8_0 N = 2 at
+    // 30000 x 2048 14.4 us, with larger ones 17.9; at 20000 x 4096 17.5 against
+    // 18.9.  Below that where larger ones measured slower (larger -> four, us): N = 2
+    // Q8_0 6144 x 2048 5.84 -> 5.42, Q2_0 4096 x 2048 4.96 -> 4.48, Q4_0 4096 x 1024
+    // 4.30 -> 3.96, Q6_K 12288 x 2048 8.16 -> 7.60; N = 5 Q6_K 10240 x 2048 17.0 ->
+    // 13.9, Q8_0 4096 x 1024 6.27 -> 5.73, Q2_0 6144 x 2048 8.99 -> 8.41; N = 4 Q2_0
+    // 4096 x 2048 6.95 -> 5.97; N = 3 F16 12288 x 2048 12.0 -> 10.3.
+    constexpr bool lean = F == Q8_0 || F == Q2_0 || F == Q4_0 || F == IQ4_NL || F == Q6_K;
+    const bool shorts = K <= 2048 && M >= 16ull * c->cus &&
+                        ((lean && (NC == 2 || (F == Q6_K && NC != 4) || (F != Q2_0 && K <= 1024))) ||
+                         (F == Q2_0 && K > 1024 && M <= 32ull * c->cus && (NC < 5 || M >= 20ull * c->cus)) ||
+                         ((F == F16 || F == BF16) && NC >= 3 && M >= 40ull * c->cus) ||
+                         (F == F32 && K <= 1024 && M >= 40ull * c->cus));
+    // (F32 rows that four wavefronts spread evenly: 8192 x 8192 N = 3 58.2 -> 51.3)
+    const bool even = F == F32 && K >= 3072 && M % (32ull * c->cus) == 0;
+    const bool many = !c->gemv_s && (shorts || even || (K <= 4096 && M > 64ull * c->cus));
     for (const auto &f : forms) {
         const uint32_t W = f[0], S = f[1], rows = W / S * GV_SLOTS * R;
         if (many && (W > 4 || S > 1)) continue;
         if (F == Q6_K && steps < 2 * S) continue;  // (2048 x 2048, N = 3: 5.5 us without a split, 5.9 with)
         if (W > MAXW || (c->gemv_s && S != std::min<uint32_t>(c->gemv_s, 4))) continue;
-        const uint32_t fit = (uint32_t)std::min<size_t>(c->max_lds / (xb + 1024), (MAXW == 8 ? 8u : 12u) / W);
+        const uint32_t fit = (uint32_t)std::min<size_t>(c->max_lds / (xb + 1024), MAXW / W);
         const uint32_t slots = std::max(1u, fit), cus = std::max(1u, c->cus);
         const uint64_t wgs = (M + rows - 1) / rows, full = wgs / ((uint64_t)cus * slots);
         const uint32_t rest = (uint32_t)((wgs - full * cus * slots + cus - 1) / cus);
@@ -238,7 +252,7 @@ GemvPlan plan_gemv(const okf_ctx *c, uint64_t M, uint32_t K) {
     return best;
 }
 
-template <int F, int NC, int S, bool SILU, int DX = 0>
+template <int F, int NC, int S, bool SILU, int DX = 0, uint32_t MW = gemv_max_waves<F, NC>()>
 void launch_gemv_s(okf_ctx *c, const GemvCall *calls, int n, uint64_t rb, uint32_t K,
                    uint32_t cunits, size_t lds, bool pair = false, uint32_t waves = 4) {
     // Q2_0 and Q8_0 at N = 1: a three-deep ring when a wavefront runs three
@@ -249,8 +263,10 @@ void launch_gemv_s(okf_ctx *c, const GemvCall *calls, int n, uint64_t rb, uint32
         const uint32_t steps = (K / unit_weights<F>() + GV_L * S - 1) / (GV_L * S);
         if (steps >= 3) return launch_gemv_s<F, NC, S, SILU, 3>(c, calls, n, rb, K, cunits, lds, pair, waves);
     }
+    if constexpr (S == 1 && MW > 4)
+        if (waves == 4) return launch_gemv_s<F, NC, S, SILU, DX, 4>(c, calls, n, rb, K, cunits, lds, pair, waves);
     constexpr int R = gemv_rows<F, NC>(), D = DX ? DX : 2;
-    const void *fn = (const void *)gemv_kernel<F, NC, R, D, S, SILU>;
+    const void *fn = (const void *)gemv_kernel<F, NC, R, D, S, SILU, MW>;
     static std::atomic<uint64_t> attr{0};  // devices that have the attribute set
     set_lds_attr(c, fn, attr);
     const uint32_t rows_per_wg = (waves / S) * GV_SLOTS * R;
@@ -273,7 +289,7 @@ void launch_gemv_s(okf_ctx *c, const GemvCall *calls, int n, uint64_t rb, uint32
     // the tables the compute reads: IQ2_XXS's LDS rows (copied from c->tab),
     // or the grid formats' device-memory grids
     const u32x4 *tabs = itab_rows(F) ? c->tab8 + itab_at(F) : grid_fmt(F) ? (const u32x4 *)(c->grids + gt_off(F)) : c->tab8;
-    hipLaunchKernelGGL((gemv_kernel<F, NC, R, D, S, SILU>), dim3(total), dim3(64 * waves), lds, c->stream,
+    hipLaunchKernelGGL((gemv_kernel<F, NC, R, D, S, SILU, MW>), dim3(total), dim3(64 * waves), lds, c->stream,
                        g, rb, K, tabs, cunits);
 }
 

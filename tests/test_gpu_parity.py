@@ -1236,7 +1236,8 @@ def test_gemv_superblock_edges(enc_sb, t, M, K):
 # ------------------------------------------------------------------ gemv_kernel, 2..5 columns
 # Workgroups of 4 to 12 wavefronts, K split over 1, 2 or 4 of them (forced by
 # OKF_GEMV_S; None: the planned one): one row, rows that fill no workgroup, fewer
-# steps than parts, x staged in chunks (K = 17408), Q4_K / Q5_K columns in two
+# steps than parts, x staged in chunks (K = 17408), many short rows (four
+# wavefronts, an instance of their own), Q4_K / Q5_K columns in two
 # launches.  Against the oracle at the matvec gate.
 @pytest.fixture(scope="module", params=[None, "1", "2", "4"], ids=lambda v: f"split{v or '_planned'}")
 def enc_gemv_s(request):
@@ -1252,7 +1253,7 @@ def enc_gemv_s(request):
 
 
 @pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K, Q3_K, Q8_0, Q2_0, IQ3_XXS, F32, F16], ids=lambda t: NAMES[t])
-@pytest.mark.parametrize("M,K", [(1, 256), (2003, 768), (1025, 2304), (37, 9216), (261, 17408)])
+@pytest.mark.parametrize("M,K", [(1, 256), (2003, 768), (1025, 2304), (37, 9216), (261, 17408), (16401, 768)])
 def test_gemv_columns_workgroups(enc_gemv_s, t, M, K):
     say("columns", NAMES[t], M, K)
     w, X = weights(t, M, K, 31), acts(5, K, 32)

@@ -121,6 +121,19 @@ def test_superblock_matvec_iq2_xxs(fake, M, K, sb):
     assert [v["name"] for v in r["launches"]] == ["gemv_sb_kernel" if sb else "gemv_kernel"]
 
 
+# ------------------------------------------------------------------ several columns
+# Many short rows: four wavefronts without a split, in the instance whose
+# registers are those of four (a larger workgroup's cost F32, N = 2, a fifth).
+@pytest.mark.parametrize("fmt,M,K,N", [("f32", 151936, 2048, 2), ("q8_0", 248320, 1024, 2), ("q8_0", 6144, 2048, 2),
+                                       ("q2_0", 4096, 2048, 2), ("q6_k", 10240, 2048, 5), ("q4_0", 4096, 1024, 3),
+                                       ("f16", 12288, 2048, 3), ("q2_0", 6144, 2048, 5)])
+def test_columns_of_many_short_rows(fake, fmt, M, K, N):
+    (r,) = fakehip.run(fake, [["gemm", fmt, M, K, N]])
+    (v,) = r["launches"]
+    f, nc, rows, depth, split, silu, most = v["args"]
+    assert (v["name"], nc, v["block"], split, most) == ("gemv_kernel", N, 256, 1, 4)
+
+
 # ------------------------------------------------------------------ RMSNorm
 # Threads a row: short rows past one a CU keep 256 (a head's norm over 128
 # values took 25.1 us for 16384 rows on 512 threads, 14.7 on 256).
