@@ -803,7 +803,7 @@ inline MmPlan plan_mm(const okf_ctx *c, int type, uint32_t K, uint32_t M, uint32
     };
     if (force[1] || (c->gemm_ks == 0 && (N < 256 || type == Q4_K))) {
 #define OKF_CONSIDER(a, b)                      \
-    for (uint32_t ks = 1; ks <= 4; ks *= 2) consider(0, a, b, ks);
+    for (uint32_t ks = 1; ks <= (c->gemm_split ? 4u : 1u); ks *= 2) consider(0, a, b, ks);
         OKF_FEW(OKF_CONSIDER)
 #undef OKF_CONSIDER
     }

@@ -80,8 +80,7 @@ def test_one_range_is_planned_as_one(fake, fmt, M, K, N, how):
     assert tile_launch(free)[3] > 1 and "gemm_ksum_kernel" in [v["name"] for v in free["launches"]]
     assert tile_launch(got)[3] == 1 and "gemm_ksum_kernel" not in [v["name"] for v in got["launches"]]
     assert tile_launch(got)[2] > tile_launch(free)[2]
-    if N >= 256 and fmt != "q4_k":  # (gemm_few_kernel is not planned: OKF_GEMM_SPLIT=0 plans one range of the same)
-        assert tile_launch(got) == tile_launch(one)
+    assert tile_launch(got) == tile_launch(one)  # (OKF_GEMM_SPLIT=0 plans one range of both kernels)
 
 
 # With room for some of the ranges, as many as fit.
