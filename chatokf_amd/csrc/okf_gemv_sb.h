@@ -264,8 +264,11 @@ __device__ __forceinline__ uint32_t sb_dw(const uint32_t (&c)[ND], uint32_t off)
     return (off & 3) == 0 ? c[i] : __builtin_amdgcn_alignbyte(c[i + 1], c[i], off & 3);
 }
 // The dwords of a superblock's registers, each a value of its own.  (Taken
-// from the loaded vectors where they are used, hipcc 7.2 -O3 gave the register
-// of IQ4_XS's dword 32 to an address while it was still to be read.)
+// from the loaded vectors where they are used, IQ4_XS's 8-byte tail met an
+// error of hipcc 7.2: its si-form-memory-clauses pass keeps no live range for the
+// first half of the load, -verify-machineinstrs says "No live subrange at use",
+// and the register was given to an address before dword 32 was read.  As values
+// of their own all kernels pass the verifier; tests/test_codegen.py.)
 template <int NL>
 __device__ __forceinline__ void sb_split(const u32x4 (&c)[NL], uint32_t (&d)[4 * NL]) {
 #pragma unroll
