@@ -112,6 +112,17 @@ def test_superblock_matvec_rows(fake, fmt):
     assert sb == 2 * [K <= 20480 for K in ks]
 
 
+# Gate and up paired: an even number of rows whose items fill one round of the
+# 256 lanes.
+@pytest.mark.parametrize("fmt,K", [("q4_k", 3072), ("q5_k", 3072), ("q5_k", 7168), ("iq4_xs", 3072), ("q5_k", 6912)])
+def test_paired_superblock_rows(fake, fmt, K):
+    M = 40320
+    (r,) = fakehip.run(fake, [["gate_up", fmt, M, K]])
+    (k,) = [v for v in r["launches"] if v["name"] == "gemv_sb_kernel"]
+    rows = 2 * -(-M // k["grid"][0])
+    assert k["block"] == 256 and 200 < rows * (K // 256) <= 256
+
+
 # IQ2_XXS: tall matrices of short rows too (248320 x 1024 33.0 us on gemv_kernel, 26.6).
 @pytest.mark.parametrize("M,K,sb", [(248320, 1024, True), (120000, 2048, True), (60000, 512, True), (60000, 2048, False),
                                     (6144, 2048, False), (17408, 5120, True), (30000, 256, False)])
