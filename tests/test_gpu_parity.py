@@ -1059,11 +1059,12 @@ def test_injected_fault_launches_nothing(enc):
 # ------------------------------------------------------------------ embedding gather
 @pytest.mark.parametrize("t", [Q8_0, Q2_0, Q4_K, IQ2_XXS, Q4_0, IQ4_NL, Q5_K, Q6_K, IQ4_XS, IQ2_XS, IQ2_S,
                                IQ3_XXS, IQ3_S, IQ1_S, IQ1_M, Q2_K, Q3_K, F32, F16, BF16], ids=lambda t: NAMES[t])
-def test_embed_batch_bit_exact(enc, t):
+@pytest.mark.parametrize("N", [8, 2, 1])  # (one row: 64 units, stored without LDS)
+def test_embed_batch_bit_exact(enc, t, N):
     # embedBatch (MetalEnc.swift:1096-1146) vs the oracle's dequant of each row
     M, K = 300, 2048
     w = weights(t, M, K, 91)
-    ids = np.array([0, 299, 17, 17, 150, 1, 298, 64], np.int32)
+    ids = np.array([0, 299, 17, 17, 150, 1, 298, 64], np.int32)[-N:]
     out = torch.full((len(ids), K), float("nan"), device="cuda")
     enc.embed_batch(ok.QuantTensor(dev(w), K, M, t), dev(ids), len(ids), out)
     got = host(out)
