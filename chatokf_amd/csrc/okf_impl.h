@@ -448,23 +448,43 @@ void launch_sb_t(okf_ctx *c, const GemvGroup &g, uint32_t total, uint64_t rb, ui
 // IQ4_NL 17408 x 5120 (348 K) 14.9 -> 15.3, 60000 x 2048 18.7 -> 17.0, 5120 x 17408
 // 22.0 -> 17.2; IQ2_XXS 2048 x 2048 4.1 -> 7.6, 12288 x 3584 9.8 -> 11.4, 17408 x 5120
 // 14.9 -> 13.9, 60000 x 2048 16.2 -> 17.6, 120000 x 1536 25.0 -> 22.0, 248320 x 1024
-// 33.0 -> 26.6, 248320 x 4096 89.5 -> 83.1, 60000 x 512 10.6 -> 8.9.  Gate and up paired (okf_ffn, H x D):
+// 33.0 -> 26.6, 248320 x 4096 89.5 -> 83.1, 60000 x 512 10.6 -> 8.9.  okf_ffn (gate
+// and up paired, and down; H x D; IQ4_XS's gain is down's):
 // 6144 x 2048 Q4_K 10.6 -> 10.8, Q5_K 11.6 -> 11.9, Q8_0 12.5 -> 13.1; 7168 x 3584 Q4_K
 // 16.4 -> 16.0, Q5_K 20.7 -> 17.7, IQ4_NL 18.3 -> 19.7; 17408 x 5120 Q4_K 37.2 -> 35.8,
 // Q5_K 55.6 -> 41.9, IQ4_XS 50.6 -> 44.9, IQ4_NL 55.6 -> 45.3, Q4_0 52.6 -> 35.7, Q8_0
 // 78.7 -> 59.7, IQ2_XXS 41.3 -> 41.9.
+// From a sweep of K = 512 .. 17408 and 20 K .. 700 K superblocks, weights from HBM
+// (gemv_kernel = 1): short rows of whole 1024s, which leave no lane of gemv_kernel
+// idle: IQ4_XS 4096 x 6144 1.12, 5400 x 6144 1.14 (2048 x 12250 0.98), Q8_0 4096 x 6144 and
+// 3060 x 8192 1.03; paired, rows of both, IQ4_XS 34944 x 5120 1.03, 12500 x 7168 1.07, 25000 x
+// 7168 1.10 (26680 x 4608 0.92), Q4_K 17136 x 7168 1.08, 15000 x 8192 1.10 (35000 x 5120 0.95), IQ4_NL
+// 25000 x 7168 1.06.  Long rows with one to one and a half 32-row workgroups a CU, whose
+// second round is mostly empty: Q8_0 10000 x 10240 1.05, 9803 x 14336 1.15; paired IQ4_XS 8320 x
+// 9216 1.12, 10240 x 17408 1.06 (Q4_K, Q5_K, Q4_0 0.7 to 1.05).
 template <int F>
-bool sb_auto(uint64_t rows, uint32_t K, bool pair) {
-    const uint64_t n = rows * (K / 256);  // (paired: of both matrices)
-    const bool lng = K > 8192;
-    if (pair) return n >= (F == Q4_K || F == Q5_K || F == IQ4_XS ? 190000u : 380000u);
+bool sb_auto(uint64_t rows, uint32_t K, bool pair, uint32_t cus) {
+    const uint32_t nsb = K / 256;
+    const uint64_t n = rows * nsb;  // (paired: of both matrices)
+    const bool lng = K > 8192, tail = lng && rows > 32ull * cus && rows <= 48ull * cus, whole = K % 1024 == 0;
+    if (pair) {
+        switch (F) {
+            case Q4_K: return n >= 190000 && (lng || K <= 6144 || !whole);
+            case IQ4_XS: return n >= 190000 && (lng ? !tail : K < 5120 || !whole);
+            case Q5_K: return n >= 190000;
+            // (the pair's rows leave a tenth of the 256 lanes idle)
+            case IQ4_NL: return n >= 380000 && (lng || !whole || (256 / nsb & ~1u) * nsb >= 230);
+            default: return n >= 380000;
+        }
+    }
     switch (F) {
         case Q4_K: return lng || n >= 30000;
         case Q5_K: return n >= 30000;
         case IQ2_XXS: return (n >= 100000 && K >= 5120) || rows >= 120000 || (K <= 512 && rows >= 50000);
         case Q4_0: return n >= (lng ? 96000u : 300000u);
         case IQ4_NL: return n >= (lng ? 96000u : 400000u);
-        default: return n >= 96000;  // Q8_0, IQ4_XS
+        case IQ4_XS: return n >= (lng || K <= 5120 || !whole ? 96000u : 140000u);
+        default: return n >= (lng || K <= 5120 || !whole ? 96000u : 110000u) && !tail;  // Q8_0
     }
 }
 
@@ -483,7 +503,7 @@ bool launch_gemv_sb(okf_ctx *c, const GemvCall *calls, int n, uint64_t rb, uint3
         if (c->gemv_sb == 0 || K % 256) return false;
         uint32_t M = 0;
         for (int i = 0; i < n; i++) M += calls[i].M;
-        if (c->gemv_sb < 0 && !sb_auto<F>(M, K, pair)) return false;
+        if (c->gemv_sb < 0 && !sb_auto<F>(M, K, pair, c->cus)) return false;
         const bool lng = nsb > 32;
         if (F == IQ2_XXS && (lng || pair)) return false;  // (long or paired rows: gemv_kernel is no slower)
         uint32_t T = c->gemv_sb_t ? (uint32_t)c->gemv_sb_t : lng ? 512 : 256;

@@ -123,6 +123,21 @@ def test_paired_superblock_rows(fake, fmt, K):
     assert k["block"] == 256 and 200 < rows * (K // 256) <= 256
 
 
+# Where gemv_sb_kernel is the slower one: some short rows of whole 1024s, and one to
+# one and a half 32-row workgroups a CU of long rows (Q8_0; IQ4_XS paired).
+@pytest.mark.parametrize("call,fmt,M,K,sb", [
+    ("gemv", "q8_0", 9803, 14336, False), ("gemv", "q8_0", 8192, 14336, True), ("gemv", "q8_0", 12289, 14336, True),
+    ("gemv", "q4_k", 9803, 14336, True), ("gemv", "iq4_xs", 4096, 6144, False), ("gemv", "iq4_xs", 4096, 6400, True),
+    ("gemv", "iq4_xs", 17408, 5120, True), ("gemv", "q8_0", 4096, 6144, False), ("gemv", "q8_0", 12250, 2048, True),
+    ("gate_up", "iq4_xs", 17408, 5120, False), ("gate_up", "iq4_xs", 13340, 4608, True),
+    ("gate_up", "iq4_xs", 5120, 17408, False), ("gate_up", "iq4_xs", 8192, 17408, True),
+    ("gate_up", "q4_k", 8704, 7168, False), ("gate_up", "q4_k", 8704, 6912, True), ("gate_up", "q4_k", 17408, 5120, True),
+    ("gate_up", "iq4_nl", 8704, 7168, False), ("gate_up", "iq4_nl", 17408, 5120, True), ("gate_up", "q5_k", 8704, 7168, True)])
+def test_superblock_matvec_lines(fake, call, fmt, M, K, sb):
+    (r,) = fakehip.run(fake, [[call, fmt, M, K]])
+    assert [v["name"] for v in r["launches"]] == ["gemv_sb_kernel" if sb else "gemv_kernel"]
+
+
 # IQ2_XXS: tall matrices of short rows too (248320 x 1024 33.0 us on gemv_kernel, 26.6).
 @pytest.mark.parametrize("M,K,sb", [(248320, 1024, True), (120000, 2048, True), (60000, 512, True), (60000, 2048, False),
                                     (6144, 2048, False), (17408, 5120, True), (30000, 256, False)])
