@@ -794,7 +794,9 @@ inline bool mm_instance(int kind, int fm, int fn) {
 //  few: a wavefront's step takes 0.1 + w fm + 0.2 fn + 0.06 fm fn, times the
 //    workgroups that share a CU, and 2.5 besides (6144 x 2048, N = 19: 7.7 us
 //    against 11.1 for many; N = 48: 10.3 against 13.4); w: 0.25, more for the
-//    formats whose pieces take many loads;
+//    formats whose pieces take many loads; past one workgroup a CU no less than
+//    0.55 fm fn each, the sum of its wavefronts' tiles (IQ4_NL 151936 x 1024, N = 33:
+//    fm 2, fn 4 108 us, many with fm 8 72; Q4_K 65536 x 512 36 and 21);
 //  K ranges: the partial tiles written and read at 5 TB/s, and a launch.
 // From 256 tokens on the formats but Q4_K take only many, whose sums are in
 // gemm_mfma_kernel's order (few takes K in another order within 128).
@@ -819,7 +821,10 @@ inline MmPlan plan_mm(const okf_ctx *c, int type, uint32_t K, uint32_t M, uint32
         const uint64_t wgs = up(M, 16 * fm) * up(N, (kind ? 128 : 16) * fn) * ks;
         double t = (double)N * M * 4 / 5e6 + (ks > 1 ? 2.5 + (double)ks * N * M * 8 / 5e6 : 0);
         if (kind) t += (double)up(wgs, cus) * (per * fm * (0.15 + 0.17 * fn) + 5);
-        else t += 2.5 + std::max(1.0, (double)wgs / cus) * (double)up(per, 4) * (0.1 + w * fm + 0.2 * fn + 0.06 * fm * fn);
+        else {
+            const double wg = (double)up(per, 4) * (0.1 + w * fm + 0.2 * fn + 0.06 * fm * fn), more = (double)wgs / cus - 1;
+            t += 2.5 + wg + std::max(0.0, more) * std::max(wg, 0.55 * fm * fn);
+        }
         if (best == 0 || t < best) {
             best = t;
             p = MmPlan{kind, fm, fn, ks, per * unit};

@@ -100,6 +100,16 @@ def test_many_tokens_fit_the_grid(fake, M, K, N):
         assert max(v["grid"][1:]) <= 65535 and v["grid"][0] * v["block"] < 1 << 32
 
 
+# Tall matrices of short rows: a few-token workgroup there is mostly the sum of its
+# wavefronts' tiles (Q4_K 65536 x 512, N = 33 36 us, on gemm_many_kernel 21).
+@pytest.mark.parametrize("fmt,M,K,N,few", [("q4_k", 65536, 512, 33, False), ("q4_0", 151936, 1024, 64, False),
+                                           ("iq4_nl", 151936, 1024, 33, False), ("q4_k", 65536, 512, 17, True),
+                                           ("q4_k", 6144, 2048, 19, True), ("q4_k", 1000, 512, 64, True)])
+def test_tall_short_rows(fake, fmt, M, K, N, few):
+    (r,) = fakehip.run(fake, [["gemm", fmt, M, K, N]])
+    assert tile_launch(r)[0] == ("gemm_few_kernel" if few else "gemm_many_kernel")
+
+
 # ------------------------------------------------------------------ superblock matvec
 # gemv_sb_kernel keeps a lane's staged activations in registers: up to five
 # rounds (K = 20480); longer rows stay with the other matvecs, alone and paired.
