@@ -174,7 +174,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_few_kernel(const uint8_t *__rest
 // LDS half: the 16 bytes of K step kb (of 8), row tile i, octet g (of 4) and
 // row r (of 16) are at 1024 (FM kb + i) + 256 g + 16 (r ^ mc_swz(kb, g)), so a
 // read is 1 KB of which each lane takes 16 bytes, every bank the same number
-// of times.  A write instruction's 16 lanes are 8 pieces of two rows, whose
+// of times (SQ_LDS_BANK_CONFLICT counts one cycle a read, a sixth of the LDS's).  A write instruction's 16 lanes are 8 pieces of two rows, whose
 // octets lie in different K steps or octet columns, all at the same place of
 // the 256 bytes of all banks but for the exclusive or, which takes the pieces'
 // two rows to 16 different places.  (Unswizzled, the writes took a third of the

@@ -310,8 +310,8 @@ void launch_wide_sp(okf_ctx *c, const GemvCall &call, uint64_t rb, uint32_t K, u
 // Where the one-workgroup-per-CU kernel measured faster on MI355X than the
 // many-workgroup one (A/B in one process, configuration shapes): IQ2_XXS
 // with 2..5 columns (conflict-free tables; 28.2 -> 22.5 us at N = 4),
-// Q4_0 / IQ4_NL and long-K Q2_0 with 4..5 columns, and the long-K Q4_K
-// matvec (5120 x 17408: 16.0 -> 15.4 us).
+// Q4_0 / IQ4_NL and long-K Q2_0 with 4..5 columns, and the Q4_K matvec of rows
+// past gemv_sb_kernel's 20480 (8192 x 24576: 45.2 -> 24.9 us).
 template <int F, int NC>
 bool wide_auto(const okf_ctx *c, uint32_t M, uint32_t K) {
     if (M < 8 * c->cus) return F == Q2_0 && NC >= 4 && K >= 4096;
@@ -897,9 +897,11 @@ int launch_gemm(okf_ctx *c, const uint8_t *W, uint64_t rb, uint32_t K, uint32_t 
     note_capture(c, !st, part != nullptr, false);
     const u32x4 *tab = dq_tab_rows<F>() ? c->tab8 : nullptr;
     if (st) {
-        dim3 grid((N + GB_N - 1) / GB_N, (M + GB_M - 1) / GB_M, ks);
-        hipLaunchKernelGGL((gemm_mfma_kernel<F>), grid, dim3(256), 0, c->stream, W, rb, K, M, X, N, Y, c->grid, c->grids,
-                           kper, part);
+        if constexpr (F != Q4_K) {
+            dim3 grid((N + GB_N - 1) / GB_N, (M + GB_M - 1) / GB_M, ks);
+            hipLaunchKernelGGL((gemm_mfma_kernel<F>), grid, dim3(256), 0, c->stream, W, rb, K, M, X, N, Y, c->grid,
+                               c->grids, kper, part);
+        }
     } else {
         half8 *xt = (half8 *)c->xh;
         hipLaunchKernelGGL(x_to_octets_kernel, dim3((N + 15) / 16, (K / 8 + 63) / 64), dim3(256), 0, c->stream, X, N, K / 8,

@@ -179,11 +179,12 @@ void build_iq2_xs_s_tables8(uint32_t *t, const uint64_t *grid, int n, const uint
 enum class Path { Auto, Tile };
 
 // N > 5 as consecutive narrow launches of up to narrow_cols columns, while N
-// <= narrow_max: their results keep X in fp32, the tile's round it to fp16.  The
-// bounds lie where the chunks met gemm_mfma_kernel (the tile kernel of a context
-// without scratch; gemm_few_kernel is faster at most of them, e.g. Q4_K
-// 5120 x 17408, N = 12, 28.9 us, but would round those N's activations).  MI355X,
-// chunks against gemm_mfma_kernel with its K split (us, N = 6 / 8 / 12 / 16): 2048 x 2048 Q8_0 chunks 11.3 / 12.4 / 18.2 / 24.6, tile 11.5 / 11.4 /
+// <= narrow_max: for precision, since their results keep X in fp32 where the tile's
+// round it to fp16.  The bounds lie where the chunks met gemm_mfma_kernel (the tile
+// kernel of a context without scratch); gemm_few_kernel is faster at most of them, e.g.
+// Q4_K 5120 x 17408, N = 12, 28.9 us, but would round those N's activations.  MI355X,
+// chunks against gemm_mfma_kernel with its K split (us, N = 6 / 8 / 12 / 16): 2048 x
+// 2048 Q8_0 chunks 11.3 / 12.4 / 18.2 / 24.6, tile 11.5 / 11.4 /
 // 11.6 / 11.6; Q6_K 11.1 / 12.5 against 12.3 / 12.6; IQ4_XS 11.2 / 12.0 /
 // 18.2 against 14.0 / 14.1 / 14.4; Q4_0, Q4_K, IQ2_XXS, IQ3_XXS, Q2_K and
 // Q2_0 (2048 x 6144) tile from N = 6.  17408 x 5120: IQ2_XXS 35.4 / 36.8 /

@@ -167,7 +167,7 @@ int okf_silu_mul(okf_ctx *ctx, float *a, const float *b, uint32_t n);
  * N > 5 -> MFMA tile GEMM (gemmTiled / iqGemmTiled, :354-400; where the
  * tiles do not fill the CUs K may be split over workgroups, partials added in
  * K order), except that a small N past 5 (up to a per-format bound, 5..16
- * columns, where measured faster than the tile) runs as consecutive narrow
+ * columns, so that X keeps fp32, which the tile rounds to fp16) runs as consecutive narrow
  * launches of 4 or 5 columns (for IQ2_XXS, and for every other K-quant and
  * i-quant format but Q6_K and IQ4_NL with K <= 6144 and M >= 4096, from N =
  * 5 on, in 4-column launches).  The results are the narrow kernels' for
