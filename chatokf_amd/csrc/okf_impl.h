@@ -457,8 +457,9 @@ void launch_sb_t(okf_ctx *c, const GemvGroup &g, uint32_t total, uint64_t rb, ui
 // From a sweep of K = 512 .. 17408 and 20 K .. 700 K superblocks, weights from HBM
 // (gemv_kernel = 1): short rows of whole 1024s, which leave no lane of gemv_kernel
 // idle: IQ4_XS 4096 x 6144 1.12, 5400 x 6144 1.14 (2048 x 12250 0.98), Q8_0 4096 x 6144 and
-// 3060 x 8192 1.03; paired, rows of both, IQ4_XS 34944 x 5120 1.03, 12500 x 7168 1.07, 25000 x
-// 7168 1.10 (26680 x 4608 0.92), Q4_K 17136 x 7168 1.08, 15000 x 8192 1.10 (35000 x 5120 0.95), IQ4_NL
+// 3060 x 8192 1.03; paired, rows of both, IQ4_XS 12500 x 7168 1.07, 25000 x 7168
+// 1.10 (26680 x 4608 0.92; 34944 x 5120 1.03, but 0.97 where the weights are in the last-level
+// cache), Q4_K 17136 x 7168 1.08, 15000 x 8192 1.10 (35000 x 5120 0.95), IQ4_NL
 // 25000 x 7168 1.06.  Long rows with one to one and a half 32-row workgroups a CU, whose
 // second round is mostly empty: Q8_0 10000 x 10240 1.05, 9803 x 14336 1.15; paired IQ4_XS 8320 x
 // 9216 1.12, 10240 x 17408 1.06 (Q4_K, Q5_K, Q4_0 0.7 to 1.05).
@@ -469,8 +470,8 @@ bool sb_auto(uint64_t rows, uint32_t K, bool pair, uint32_t cus) {
     const bool lng = K > 8192, tail = lng && rows > 32ull * cus && rows <= 48ull * cus, whole = K % 1024 == 0;
     if (pair) {
         switch (F) {
-            case Q4_K: return n >= 190000 && (lng || K <= 6144 || !whole);
-            case IQ4_XS: return n >= 190000 && (lng ? !tail : K < 5120 || !whole);
+            case Q4_K:
+            case IQ4_XS: return n >= 190000 && (lng ? F == Q4_K || !tail : K <= 6144 || !whole);
             case Q5_K: return n >= 190000;
             // (the pair's rows leave a tenth of the 256 lanes idle)
             case IQ4_NL: return n >= 380000 && (lng || !whole || (256 / nsb & ~1u) * nsb >= 230);

@@ -139,7 +139,7 @@ def test_paired_superblock_rows(fake, fmt, K):
     ("gemv", "q8_0", 9803, 14336, False), ("gemv", "q8_0", 8192, 14336, True), ("gemv", "q8_0", 12289, 14336, True),
     ("gemv", "q4_k", 9803, 14336, True), ("gemv", "iq4_xs", 4096, 6144, False), ("gemv", "iq4_xs", 4096, 6400, True),
     ("gemv", "iq4_xs", 17408, 5120, True), ("gemv", "q8_0", 4096, 6144, False), ("gemv", "q8_0", 12250, 2048, True),
-    ("gate_up", "iq4_xs", 17408, 5120, False), ("gate_up", "iq4_xs", 13340, 4608, True),
+    ("gate_up", "iq4_xs", 17408, 5120, True), ("gate_up", "iq4_xs", 12500, 7168, False),
     ("gate_up", "iq4_xs", 5120, 17408, False), ("gate_up", "iq4_xs", 8192, 17408, True),
     ("gate_up", "q4_k", 8704, 7168, False), ("gate_up", "q4_k", 8704, 6912, True), ("gate_up", "q4_k", 17408, 5120, True),
     ("gate_up", "iq4_nl", 8704, 7168, False), ("gate_up", "iq4_nl", 17408, 5120, True), ("gate_up", "q5_k", 8704, 7168, True)])
