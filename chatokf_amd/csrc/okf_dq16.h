@@ -7,13 +7,14 @@
 // (DqRaw) are apart from the conversion (dq_piece), so that the bytes of a
 // later step are in flight while a step computes.
 //
-// Every weight is formed as fma(q, a, o) with q an exact small integer in
-// fp16 and a, o in fp32, and rounded to fp16 once (v_fma_mixlo_f16 /
-// v_fma_mixhi_f16): the fp32 product is exact for all of these formats but
-// Q4_K and Q5_K (whose fp32 sum has one more rounding of 2^-24), so the
-// result is the fp16 rounding of the weight that decode_unit gives (infinite
-// scales: dq_inf).
+// Every weight is rounded to fp16 once, from a product that is exact before
+// that, so it is the fp16 rounding of the weight that decode_unit gives: an exact
+// small integer in fp16 times an fp16 scale (dq_mul: Q8_0, Q2_0, Q4_0, IQ4_NL), or
+// fma(q, a, o) with a, o in fp32 (dq_pair, v_fma_mixlo_f16 / v_fma_mixhi_f16; Q4_K
+// and Q5_K: the fp32 sum has one more rounding of 2^-24).  Infinite scales: dq_inf.
 #pragma once
+#include <type_traits>
+
 #include "okf_common.h"
 #include "okf_decode.h"
 #include "okf_gemv.h"
@@ -146,33 +147,44 @@ __device__ __forceinline__ uint32_t dq_pair(half2v q, float a, float o) {
     const half2v r = {(_Float16)fmaf((float)q[0], a, o), (_Float16)fmaf((float)q[1], a, o)};
     return __builtin_bit_cast(uint32_t, r);
 }
-// 8 unsigned bytes (dwords b0, b1) as 1024 + byte in fp16, then fma: o
-// includes -1024 a (exact where used: a has at most 18 significant bits)
-__device__ __forceinline__ half8 dq_bytes(uint32_t b0, uint32_t b1, float a, float o) {
-    const uint32_t p0 = perm(0x64646464u, b0, 0x04010400u), p1 = perm(0x64646464u, b0, 0x04030402u);
-    const uint32_t p2 = perm(0x64646464u, b1, 0x04010400u), p3 = perm(0x64646464u, b1, 0x04030402u);
-    return __builtin_bit_cast(half8, uint4{dq_pair(__builtin_bit_cast(half2v, p0), a, o),
-                                           dq_pair(__builtin_bit_cast(half2v, p1), a, o),
-                                           dq_pair(__builtin_bit_cast(half2v, p2), a, o),
-                                           dq_pair(__builtin_bit_cast(half2v, p3), a, o)});
+// Two exact codes by a scale that is itself an fp16 value: one packed
+// multiplication rounds the exact product once (the bits of dq_pair).
+__device__ __forceinline__ uint32_t dq_mul(half2v q, _Float16 d) {
+    return __builtin_bit_cast(uint32_t, q * half2v{d, d});
+}
+__device__ __forceinline__ half2v dq_h2(uint32_t v) { return __builtin_bit_cast(half2v, v); }
+// 8 unsigned bytes (dwords b0, b1) less C, exactly in fp16 through 1024 + byte,
+// each pair through f; C < 0: as 1024 + byte
+template <int C, class Fn>
+__device__ __forceinline__ half8 dq_bytes(uint32_t b0, uint32_t b1, Fn f) {
+    auto q = [&](uint32_t b, uint32_t sel) {
+        const half2v p = dq_h2(perm(0x64646464u, b, sel));
+        if constexpr (C < 0) return f(p);
+        else return f(p + half2v{(_Float16)(-1024.0f - C), (_Float16)(-1024.0f - C)});
+    };
+    return __builtin_bit_cast(half8, uint4{q(b0, 0x04010400u), q(b0, 0x04030402u), q(b1, 0x04010400u),
+                                           q(b1, 0x04030402u)});
 }
 // 8 nibbles (one per byte of b0, b1) exactly in fp16 through
-// v_cvt_scalef32_pk_f16_fp8 (a nibble in an e4m3 byte is q 2^-9), then fma
-__device__ __forceinline__ half8 dq_nibbles(uint32_t b0, uint32_t b1, float a, float o) {
-    return __builtin_bit_cast(half8,
-                              uint4{dq_pair(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(b0, 512.0f, false), a, o),
-                                    dq_pair(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(b0, 512.0f, true), a, o),
-                                    dq_pair(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(b1, 512.0f, false), a, o),
-                                    dq_pair(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(b1, 512.0f, true), a, o)});
+// v_cvt_scalef32_pk_f16_fp8 (a nibble in an e4m3 byte is q 2^-9), each pair through f
+template <class Fn>
+__device__ __forceinline__ half8 dq_nibbles(uint32_t b0, uint32_t b1, Fn f) {
+    return __builtin_bit_cast(half8, uint4{f(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(b0, 512.0f, false)),
+                                           f(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(b0, 512.0f, true)),
+                                           f(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(b1, 512.0f, false)),
+                                           f(__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(b1, 512.0f, true))});
 }
 
-// An infinite block scale: d q + o with o = -C d would be NaN for every code
-// (inf - inf), so such a block takes d = 1 (dq_d1) and its exact codes are then
-// multiplied by the scale: +-inf, and NaN for a zero, as d times the code.  (A
-// test and a select a piece, and a branch that a wavefront of finite scales
-// passes by: over 1000 x 1024 to 5120 x 17408 and 16 to 512 tokens 0 to 1 % in the mean of
-// a format, 4.5 % at most, Q2_0 5120 x 17408, N = 48 39.9 -> 41.7 us.)  Q4_K and Q5_K
-// need none of it: their o is the block's own min; nor Q6_K, see there.
+// An infinite block scale gives +-inf, and NaN for a zero code, as in the decoders,
+// where the codes meet it without an offset.  IQ4_XS and IQ2_XXS, whose sub-block
+// scales are no fp16 values, keep the offset in the fma (a q + o with o = -C a, exact:
+// a has at most 18 significant bits), which would give NaN for all: their scale is
+// then 1 (dq_d1) and the codes are multiplied by it after, behind a branch that a
+// wavefront of finite scales passes by.  Measured against the offset in every
+// fma and no guard, the mean over 1000 x 1024 to 5120 x 17408 and 13 to 512
+// tokens: the packed multiplication Q8_0 0.981, Q2_0 0.957, Q4_0 0.975, IQ4_NL 0.968;
+// the branch IQ4_XS and IQ2_XXS 1.000 (offset taken off the codes: 1.020, 1.027); Q6_K
+// with the branch 1.033, with the offset taken off 1.006.
 __device__ __forceinline__ float dq_d1(float d) { return __builtin_isinf(d) ? 1.0f : d; }
 __device__ __forceinline__ void dq_inf(float d, half8 (&h)[4]) {
     if (__any(__builtin_isinf(d))) {
@@ -200,15 +212,16 @@ template <int F>
 __device__ __forceinline__ void dq_piece(const DqRaw<F> &r, uint32_t u, half8 (&h)[4], const uint2 *tab,
                                          const uint2 *grid, const uint8_t *gt) {
     if constexpr (F == Q8_0) {
-        const float d = dq_d1(h2f(r.d)), o = -1152.0f * d;
+        const _Float16 d = __builtin_bit_cast(_Float16, (uint16_t)r.d);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const u32x4 &q = i < 2 ? r.q0 : r.q1;
-            h[i] = dq_bytes(q[2 * (i & 1)] ^ 0x80808080u, q[2 * (i & 1) + 1] ^ 0x80808080u, d, o);
+            h[i] = dq_bytes<128>(q[2 * (i & 1)] ^ 0x80808080u, q[2 * (i & 1) + 1] ^ 0x80808080u,
+                                 [&](half2v v) { return dq_mul(v, d); });
         }
-        dq_inf(h2f(r.d), h);
     } else if constexpr (F == Q2_0) {  // code j at bits 2 (j % 16) of dword j / 16
-        const float d = dq_d1(h2f(r.d)), o = -1025.0f * d;
+        const _Float16 d = __builtin_bit_cast(_Float16, (uint16_t)r.d);
+        const half2v m = {(_Float16)-1025.0f, (_Float16)-1025.0f};
 #pragma unroll
         for (int s = 0; s < 2; s++) {
             const uint32_t dw = s ? r.q.y : r.q.x;
@@ -224,39 +237,39 @@ __device__ __forceinline__ void dq_piece(const DqRaw<F> &r, uint32_t u, half8 (&
 #pragma unroll
             for (int k = 0; k < 2; k++)
                 h[2 * s + k] = __builtin_bit_cast(
-                    half8, uint4{dq_pair(__builtin_bit_cast(half2v, p[4 * k]), d, o),
-                                 dq_pair(__builtin_bit_cast(half2v, p[4 * k + 1]), d, o),
-                                 dq_pair(__builtin_bit_cast(half2v, p[4 * k + 2]), d, o),
-                                 dq_pair(__builtin_bit_cast(half2v, p[4 * k + 3]), d, o)});
+                    half8, uint4{dq_mul(dq_h2(p[4 * k]) + m, d), dq_mul(dq_h2(p[4 * k + 1]) + m, d),
+                                 dq_mul(dq_h2(p[4 * k + 2]) + m, d), dq_mul(dq_h2(p[4 * k + 3]) + m, d)});
         }
-        dq_inf(h2f(r.d), h);
     } else if constexpr (F == Q4_0) {  // byte j: weight j (low nibble), j + 16 (high)
-        const float d = dq_d1(h2f(r.d)), o = -8.0f * d;
+        const _Float16 d = __builtin_bit_cast(_Float16, (uint16_t)r.d);
+        const half2v m = {(_Float16)-8.0f, (_Float16)-8.0f};
+        auto f = [&](half2v v) { return dq_mul(v + m, d); };
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const uint32_t v0 = r.q[2 * (i & 1)], v1 = r.q[2 * (i & 1) + 1];
-            h[i] = i < 2 ? dq_nibbles(v0 & 0x0F0F0F0Fu, v1 & 0x0F0F0F0Fu, d, o)
-                         : dq_nibbles((v0 >> 4) & 0x0F0F0F0Fu, (v1 >> 4) & 0x0F0F0F0Fu, d, o);
+            h[i] = i < 2 ? dq_nibbles(v0 & 0x0F0F0F0Fu, v1 & 0x0F0F0F0Fu, f)
+                         : dq_nibbles((v0 >> 4) & 0x0F0F0F0Fu, (v1 >> 4) & 0x0F0F0F0Fu, f);
         }
-        dq_inf(h2f(r.d), h);
     } else if constexpr (F == IQ4_NL || F == IQ4_XS) {
-        float d, a;
+        auto put = [&](auto cc, auto f) {
+            constexpr int C = decltype(cc)::value;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint32_t v0 = r.q[2 * (i & 1)], v1 = r.q[2 * (i & 1) + 1];
+                h[i] = i < 2 ? dq_bytes<C>(iq4_levels_u(v0 & 0x0F0F0F0Fu), iq4_levels_u(v1 & 0x0F0F0F0Fu), f)
+                             : dq_bytes<C>(iq4_levels_u((v0 >> 4) & 0x0F0F0F0Fu), iq4_levels_u((v1 >> 4) & 0x0F0F0F0Fu), f);
+            }
+        };
         if constexpr (F == IQ4_NL) {
-            d = h2f(r.d);
-            a = dq_d1(d);
+            const _Float16 d = __builtin_bit_cast(_Float16, (uint16_t)r.d);
+            put(std::integral_constant<int, 128>{}, [&](half2v v) { return dq_mul(v, d); });
         } else {
             const uint32_t ib = u & 7, sh = r.hdr.x >> 16, sl = r.hdr.y >> (4 * ib);
-            d = h2f(r.hdr.x & 0xFFFF);
-            a = dq_d1(d) * (float)((int)((sl & 0xF) | (((sh >> (2 * ib)) & 3) << 4)) - 32);
+            const float d = h2f(r.hdr.x & 0xFFFF);
+            const float a = dq_d1(d) * (float)((int)((sl & 0xF) | (((sh >> (2 * ib)) & 3) << 4)) - 32), o = -1152.0f * a;
+            put(std::integral_constant<int, -1>{}, [&](half2v v) { return dq_pair(v, a, o); });
+            dq_inf(d, h);
         }
-        const float o = -1152.0f * a;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint32_t v0 = r.q[2 * (i & 1)], v1 = r.q[2 * (i & 1) + 1];
-            h[i] = i < 2 ? dq_bytes(iq4_levels_u(v0 & 0x0F0F0F0Fu), iq4_levels_u(v1 & 0x0F0F0F0Fu), a, o)
-                         : dq_bytes(iq4_levels_u((v0 >> 4) & 0x0F0F0F0Fu), iq4_levels_u((v1 >> 4) & 0x0F0F0F0Fu), a, o);
-        }
-        dq_inf(d, h);
     } else if constexpr (F == Q4_K || F == Q5_K) {
         const uint32_t j = u & 7, g = j >> 1;
         // the 6-bit scales and mins of sub-blocks 2 g, 2 g + 1
@@ -278,7 +291,7 @@ __device__ __forceinline__ void dq_piece(const DqRaw<F> &r, uint32_t u, half8 (&
             const uint32_t v1 = i < 2 ? r.q[2 * (i & 1) + 1] : r.q[2 * (i & 1) + 1] >> 4;
             const float a = i < 2 ? a0 : a1, o = i < 2 ? o0 : o1;
             if constexpr (F == Q4_K) {
-                h[i] = dq_nibbles(v0 & 0x0F0F0F0Fu, v1 & 0x0F0F0F0Fu, a, o);
+                h[i] = dq_nibbles(v0 & 0x0F0F0F0Fu, v1 & 0x0F0F0F0Fu, [&](half2v v) { return dq_pair(v, a, o); });
             } else {
                 // the fifth bit: bit 2 g (+ 1) of the qh byte
                 const uint32_t t = 2 * g + (i >> 1);
@@ -302,14 +315,7 @@ __device__ __forceinline__ void dq_piece(const DqRaw<F> &r, uint32_t u, half8 (&
             const float a = d * (float)s;
             const uint32_t b0 = ((l.x >> (4 * (i >> 1))) & 0x0F0F0F0Fu) | (((r.qh.x >> (2 * i)) & 0x03030303u) << 4);
             const uint32_t b1 = ((l.y >> (4 * (i >> 1))) & 0x0F0F0F0Fu) | (((r.qh.y >> (2 * i)) & 0x03030303u) << 4);
-            // (q - 32 exactly in fp16, so that no offset meets an infinite scale: dq_inf's
-            // branch cost a tenth here: 17408 x 5120, N = 101 54.5 us, so 50.7, unguarded 49.5)
-            const half2v m = {(_Float16)-1056.0f, (_Float16)-1056.0f};
-            auto pr = [&](uint32_t b, uint32_t sel) {
-                return dq_pair(__builtin_bit_cast(half2v, perm(0x64646464u, b, sel)) + m, a, 0.0f);
-            };
-            h[i] = __builtin_bit_cast(half8, uint4{pr(b0, 0x04010400u), pr(b0, 0x04030402u), pr(b1, 0x04010400u),
-                                                   pr(b1, 0x04030402u)});
+            h[i] = dq_bytes<32>(b0, b1, [&](half2v v) { return dq_pair(v, a, 0.0f); });
         }
     } else if constexpr (F == IQ2_XXS) {
         const float a = dq_d1(h2f(r.d)) * (0.5f + (float)(r.a.y >> 28)) * 0.25f, o = -1152.0f * a;
@@ -319,8 +325,8 @@ __device__ __forceinline__ void dq_piece(const DqRaw<F> &r, uint32_t u, half8 (&
         for (int l = 0; l < 4; l++) {
             const uint2 gv = tab[(r.a.x >> (8 * l)) & 0xFF];
             const uint2 sg = tab[256 + ((r.a.y >> (7 * l)) & 127)];
-            h[l] = dq_bytes(perm(NEG, POS, gv.x + sg.x - 0x03020100u), perm(NEG, POS, gv.y + sg.y - 0x03020100u), a,
-                            o);
+            h[l] = dq_bytes<-1>(perm(NEG, POS, gv.x + sg.x - 0x03020100u), perm(NEG, POS, gv.y + sg.y - 0x03020100u),
+                                [&](half2v v) { return dq_pair(v, a, o); });
         }
         dq_inf(h2f(r.d), h);
     } else {
